@@ -1438,9 +1438,8 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_kernel(GemmParams p) {
       // f32 C through LDS, one 32-row block of the wave tile at a time: the
       // prior C (C += A*B) is read and the result written as whole row
       // segments (F32_CPR lanes x 16 bytes per row) instead of 16-byte
-      // pieces of 32 rows. Atomic split-K adds each row segment with four
-      // buffer_atomic_add_f32, so one instruction's 64 lanes touch a few
-      // whole rows' cache lines rather than one line per lane.
+      // pieces of 32 rows. Atomic split-K adds 64 consecutive dwords per
+      // buffer_atomic_add_f32, so one instruction touches whole cache lines.
       float *base = OUT == kOutF32Partial
                         ? p.ws + (size_t)part * (size_t)p.M * (size_t)p.ws_ld
                         : reinterpret_cast<float *>(p.C);
@@ -1503,6 +1502,34 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_kernel(GemmParams p) {
               }
           }
           asm volatile("" ::: "memory");
+          if constexpr (OUT == kOutF32Atomic) {
+            // one dword per lane, 64 consecutive columns (or 2 x 32) per
+            // atomic: the atomics of a wave are served per cache line it
+            // touches, and a lane's four columns as four atomics touched
+            // every line of the block four times, a quarter of it each
+            // (1024^2 in 4 splits, K = 1024, where the atomics are nearly
+            // all of it: 54.9 us that way, 17.5 this way; K = 8200: 73.8 and
+            // 36.6). Starting each split at another row of the pass (fewer
+            // splits on one line at a time) measured 1 us slower, all splits
+            // of a tile on one XCD 0.3-2 us slower.
+            constexpr int NA = BR * T::WTN / 64; // dwords per lane per pass
+#pragma unroll
+            for (int t = 0; t < NA; ++t) {
+              const int r = (t * 64 + lane) / T::WTN; // row of the pass
+              const int c = (t * 64 + lane) % T::WTN; // column of the wave tile
+              const int cs = (c / 4) ^ ((r / T::F32_RPP) % T::F32_XOR);
+              const float v = *(const TBK_LDS float *)(wl + r * T::F32_ROWB + cs * 16 +
+                                                       (c % 4) * 4);
+              const int row = row0 + h * BR + r, acol = n0 + wn * T::WTN + c;
+              // past the edges the offset is kOob: the atomic is dropped
+              const uint32_t aoff =
+                  (row < p.M && acol < p.N)
+                      ? ((uint32_t)(row - m0) * (uint32_t)ld + (uint32_t)acol) * 4u
+                      : kOob;
+              __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(v, rc, aoff, 0, 0);
+            }
+            continue;
+          }
           // whole row segments out: segment t of the block is row t F32_RPI +
           // l / F32_CPR, in pass t / NLDH
 #pragma unroll
@@ -1519,19 +1546,12 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_kernel(GemmParams p) {
                   v[e] = epi_apply1(v[e], b[e], ea);
               }
             }
-            if constexpr (OUT == kOutF32Atomic) {
-              // past the edges off[t] is kOob: the atomics are dropped
-#pragma unroll
-              for (int e = 0; e < 4; ++e)
-                __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(v[e], rc, off[t] + 4u * e, 0, 0);
-            } else {
-              // f32 results (split-K partials, plain f32 C) are written once
-              // and not read again by this kernel: non-temporal, which leaves
-              // less dirty data in L2 for the kernel-end release (split-K 512^2
-              // x 16384: 15.7 -> 15.1 us per GEMM); C += A*B keeps the default
-              __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rc, off[t],
-                                                     0, OUT == kOutF32Partial ? kStoreNT : 0);
-            }
+            // f32 results (split-K partials, plain f32 C) are written once
+            // and not read again by this kernel: non-temporal, which leaves
+            // less dirty data in L2 for the kernel-end release (split-K 512^2
+            // x 16384: 15.7 -> 15.1 us per GEMM); C += A*B keeps the default
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rc, off[t], 0,
+                                                   OUT == kOutF32Partial ? kStoreNT : 0);
           }
         }
       }
