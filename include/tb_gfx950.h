@@ -135,7 +135,14 @@ int tb_desc_create(const tb_gemm_config *cfg, tb_gemm_desc **out);
  * already holds a sealed tb.pipeline_mainline or a lowered tb.gfx950_launch
  * is accepted as is. Operands are identity-layout memrefs, so the leading
  * dimensions are the memref row lengths. Errors carry the pass name and the
- * diagnostic (the reference's emitError text where the rule is shared). */
+ * diagnostic (the reference's emitError text where the rule is shared).
+ *
+ * A launch of a planned descriptor may run the problem on another compiled
+ * tile, or as two rectangles of C, where the planned grid would leave compute
+ * units idle (csrc/runtime/grid_split.h): every tile adds an element's
+ * products in the same order, so C is the same. The descriptor's config and
+ * kernel name stay the plan's; tb_desc_create with that config runs exactly
+ * that kernel. */
 int tb_plan_from_mlir(const char *mlir, size_t len, const char *gpu_arch,
                       tb_gemm_desc **out);
 

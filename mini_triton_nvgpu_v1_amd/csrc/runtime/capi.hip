@@ -12,6 +12,7 @@
 #include "../kernels/gemm_gfx950.h"
 #include "../plan/instances.h"
 #include "desc.h"
+#include "grid_split.h"
 
 #include <hip/hip_runtime.h>
 
@@ -212,6 +213,21 @@ int create_desc(const tb_gemm_config &c, tb_gemm_desc **out) {
   return 0;
 }
 
+void choose_parts(tb_gemm_desc *d) {
+  const std::string error = g_last_error; // a build that does not bind is no error here
+  std::vector<tb_gemm_part> parts;
+  for (const GridPart &g : split_grid(d->cfg)) {
+    tb_gemm_desc *sub = nullptr;
+    if (create_desc(g.cfg, &sub)) {
+      parts.clear();
+      break;
+    }
+    parts.push_back({std::unique_ptr<tb_gemm_desc>(sub), g.row0, g.col0});
+  }
+  d->parts = std::move(parts);
+  g_last_error = error;
+}
+
 } // namespace tbrt
 
 // ---- the scratch of tb_gemm_launch_noalloc --------------------------------
@@ -271,7 +287,10 @@ int scratch_address(hipStream_t stream, void **out) {
   return 0;
 }
 
-static int launch_impl(const tb_gemm_desc *d, const void *a, const void *b, void *c,
+int launch_kernels(const tb_gemm_desc *d, const void *a, const void *b, void *c,
+                   const void *bias, void *workspace, hipStream_t s);
+
+int launch_impl(const tb_gemm_desc *d, const void *a, const void *b, void *c,
                        const void *bias, void *workspace, void *stream, const char *who) {
   if (!d)
     return fail(std::string(who) + ": desc is NULL");
@@ -297,6 +316,30 @@ static int launch_impl(const tb_gemm_desc *d, const void *a, const void *b, void
                 std::to_string(d->workspace_bytes) + " bytes");
   if (d->workspace_bytes && reinterpret_cast<uintptr_t>(workspace) % 16)
     return fail("tb_gemm_launch: the workspace must be 16-byte aligned");
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (d->parts.empty())
+    return launch_kernels(d, a, b, c, bias, workspace, s);
+  // a part starts at whole tiles and every leading dimension is a multiple
+  // of 8 elements, so the offset operands keep the alignment checked above
+  const tb_gemm_config &cf = d->cfg;
+  const int64_t c_size = cf.c_dtype == TB_DTYPE_F16 ? 2 : 4;
+  const int64_t bias_size = cf.epi_bias == TB_EPI_BIAS_F16 ? 2 : 4;
+  for (const tb_gemm_part &part : d->parts) {
+    const int64_t r0 = part.row0, c0 = part.col0;
+    if (int rc = launch_kernels(
+            part.desc.get(), static_cast<const char *>(a) + r0 * cf.lda * 2,
+            static_cast<const char *>(b) + c0 * 2,
+            static_cast<char *>(c) + (r0 * cf.ldc + c0) * c_size,
+            bias ? static_cast<const char *>(bias) + c0 * bias_size : nullptr, nullptr, s))
+      return rc;
+  }
+  return 0;
+}
+
+// The kernel of one descriptor (and a split-K descriptor's reduction) on
+// checked operands.
+int launch_kernels(const tb_gemm_desc *d, const void *a, const void *b, void *c,
+                   const void *bias, void *workspace, hipStream_t s) {
   const tb_gemm_config &cf = d->cfg;
   tbk::GemmParams p{};
   p.A = a;
@@ -328,7 +371,6 @@ static int launch_impl(const tb_gemm_desc *d, const void *a, const void *b, void
     p.ws = reinterpret_cast<float *>(c); // plain f32 store into C
     p.ws_ld = (int)cf.ldc;
   }
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   void *args[] = {&p};
   const dim3 grid((unsigned)cf.num_programs),
       block((unsigned)(d->entry->threads ? d->entry->threads : cf.num_waves * 64));

@@ -1,0 +1,195 @@
+// The builds and rectangles a plan's launch runs (grid_split.h).
+//
+// A plan names one macro tile. Run as such, a grid of fewer tiles than CUs
+// leaves CUs idle, and a grid of a few more tiles than a multiple of 256 runs
+// a last round that is nearly empty: 24 tiles of 256x256 (1000 x 1496 x 712)
+// kept 24 of 256 CUs busy for 30 us, and 320 of them (5000 x 4096 x 4104)
+// took two rounds, the second a quarter full, 178 us. C does not depend on
+// the tile: every build adds the products of an element in the same k order
+// in f32 (bit-identical for f16 and plain f32 results; f32 C += A*B may round
+// its one addition of the prior C elsewhere). So the launch of a plan may
+// run the same problem on another tile, or cut it in two rectangles: the rows
+// (or columns) that fill whole rounds on the planned tile, and the rest on a
+// tile that spreads it over the chip.
+//
+// The choice is by time, from two measured constants per tile: a grid's
+// round of up to 256 tiles takes c0 + (K / 64) * c1(fill) us, where c1 rises
+// from `lo` (up to half the CUs: the clock is high) to `hi` (all of them:
+// the part is power-limited). Measured back to back, f16 C, K = 128 .. 4096:
+//   tile     c0    lo     hi     e.g. K = 4096, 32 / 128 / 256 tiles
+//   256x256  7.3   0.955  1.37   68.1 / 68.6 / 95.1 us
+//   256x128  4.6   0.53   0.79   38.3 / 38.8 / 56.0
+//   128x128  4.1   0.333  0.455  25.4 / 25.8 / 33.1
+//    64x128  4.1   0.32   0.37   24.1 / 24.4 / 27.9
+//    64x64   3.6   0.27   0.275  20.6 / 20.8 / 21.2
+// The 64-row tiles fit a CU two or three times, so their further rounds
+// overlap: each costs 2.6 and 1.15 us and the K part 0.32 and 0.21 us per 64
+// of K and round (512 tiles of 64x128 at K = 1024 / 4096: 16.7 / 47.5 us,
+// 1024 of 64x64 at K = 64 / 1024 / 4096: 7.9 / 19.6 / 58.9).
+// A choice has to be predicted 10% faster than the plan as it stands: the
+// constants reproduce the measured times to about 8%.
+#include "grid_split.h"
+
+#include <algorithm>
+
+namespace tbrt {
+namespace {
+
+constexpr int64_t kCus = 256;
+
+// A tile the launch may choose: its build, and its cost per round.
+struct Build {
+  int64_t bm, bn, wgm, wgn, stages;
+  int32_t mfma;
+  double c0, lo, hi;
+  // overlapping rounds: us per round after the first, and per 64 of K and
+  // round (0: rounds do not overlap)
+  double more, more_k;
+};
+const Build kBuilds[] = {
+    {256, 256, 2, 2, 2, TB_MFMA_16X16X32, 7.3, 0.955, 1.37, 0, 0},
+    {256, 128, 4, 2, 3, TB_MFMA_16X16X32, 4.6, 0.53, 0.79, 0, 0},
+    {128, 128, 2, 2, 3, TB_MFMA_16X16X32, 4.1, 0.333, 0.455, 0, 0},
+    {64, 128, 2, 4, 3, TB_MFMA_32X32X16, 4.1, 0.32, 0.37, 2.6, 0.32},
+    {64, 64, 2, 2, 3, TB_MFMA_32X32X16, 3.6, 0.27, 0.275, 1.15, 0.21},
+};
+
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+double round_us(const Build &b, int64_t tiles, double nk) {
+  const double fill = (double)tiles / kCus;
+  const double rise = std::clamp(2 * fill - 1, 0.0, 1.0);
+  return b.c0 + nk * (b.lo + rise * (b.hi - b.lo));
+}
+
+double grid_us(const Build &b, int64_t m, int64_t n, int64_t k) {
+  const int64_t tiles = ceil_div(m, b.bm) * ceil_div(n, b.bn);
+  const double nk = (double)ceil_div(k, 64);
+  if (b.more > 0 && tiles > kCus) {
+    const double rounds = (double)ceil_div(tiles, kCus);
+    return b.c0 + (rounds - 1) * b.more + nk * std::max(b.hi, rounds * b.more_k);
+  }
+  const int64_t full = tiles / kCus, rest = tiles % kCus;
+  return (double)full * round_us(b, kCus, nk) + (rest ? round_us(b, rest, nk) : 0);
+}
+
+// The build of the planned tile's shape, or null.
+const Build *build_of(const tb_gemm_config &c) {
+  for (const Build &b : kBuilds)
+    if ((b.bm == c.block_m && b.bn == c.block_n) ||
+        (b.bm == c.block_n && b.bn == c.block_m))
+      return &b;
+  return nullptr;
+}
+
+bool is_build(const tb_gemm_config &c, const Build &b) {
+  return c.block_k == 64 && c.stages == b.stages && c.num_waves == b.wgm * b.wgn;
+}
+
+// The time of the planned grid over its shape's build. A workgroup alone on
+// its CU waits for its loads on 2 stages, or issues them too slowly on 1 or 2
+// waves, once the k-loop is long (64x64, 256 tiles, K = 2048: 26.9 us on
+// 32-deep 2-stage k-tiles, 16.9 on 64-deep ones, 14.6 on 2 waves, 12.7 on
+// the build; K = 512: 6.6, 6.4, 7.0, 6.5). With several workgroups per CU
+// the stages and waves make little difference. The 256x256 tile is fastest
+// on its own build for any K from 512 (256 tiles, K = 512: 19.9 us, the
+// other builds 22.5-48).
+double over_build(const tb_gemm_config &c, const Build &b) {
+  if (is_build(c, b))
+    return 1;
+  if (b.bm == 256 && b.bn == 256)
+    return c.k >= 512 ? 1.15 : 1;
+  const int64_t tiles = ceil_div(c.m, c.block_m) * ceil_div(c.n, c.block_n);
+  return tiles <= kCus && c.k >= 1024 && (c.stages == 2 || c.num_waves < 4) ? 1.2 : 1;
+}
+
+// The finest build within 5% of the fastest: what the constants leave out
+// (fused steps, an f32 C) is per element and spreads over more CUs
+// (1000 x 1496 x 712: 8.1 us predicted on 128x128, 8.2 on 64x128; 9.9 and
+// 8.5 measured).
+const Build &fastest(int64_t m, int64_t n, int64_t k) {
+  double least = grid_us(kBuilds[0], m, n, k);
+  for (const Build &b : kBuilds)
+    least = std::min(least, grid_us(b, m, n, k));
+  const Build *best = &kBuilds[0];
+  for (const Build &b : kBuilds) // coarse to fine
+    if (grid_us(b, m, n, k) <= 1.05 * least)
+      best = &b;
+  return *best;
+}
+
+// The configuration of an m x n rectangle of c on build b: a plain grid in
+// grouped order, neighbours on one XCD once it fills the chip.
+tb_gemm_config on_build(const tb_gemm_config &c, const Build &b, int64_t m, int64_t n) {
+  tb_gemm_config r = c;
+  r.m = m;
+  r.n = n;
+  r.block_m = b.bm;
+  r.block_n = b.bn;
+  r.block_k = 64;
+  r.num_waves = b.wgm * b.wgn;
+  r.wave_grid_m = b.wgm;
+  r.wave_grid_n = b.wgn;
+  r.stages = b.stages;
+  r.mfma = b.mfma;
+  const int64_t tm = ceil_div(m, b.bm), tn = ceil_div(n, b.bn);
+  r.mapping = tm > 1 && tn > 1 ? TB_MAP_GROUPED_TILE : TB_MAP_TILE;
+  r.group_m = r.mapping == TB_MAP_GROUPED_TILE ? 8 : 1;
+  r.num_programs = tm * tn;
+  r.xcd_remap = tm * tn >= kCus ? 8 : 0;
+  return r;
+}
+
+} // namespace
+
+std::vector<GridPart> split_grid(const tb_gemm_config &c) {
+  if (c.mapping == TB_MAP_SPLIT_K)
+    return {};
+  const bool persistent =
+      c.mapping == TB_MAP_PERSISTENT_TILE || c.mapping == TB_MAP_PERSISTENT_GROUPED;
+  const int64_t tm = ceil_div(c.m, c.block_m), tn = ceil_div(c.n, c.block_n);
+  const int64_t tiles = tm * tn;
+  // a persistent plan of fewer programs than CUs asks for a part of the chip
+  if (persistent && c.num_programs < kCus)
+    return {};
+  const Build *planned = build_of(c);
+  if (!planned)
+    return {};
+  double best_us = 0.9 * over_build(c, *planned) * grid_us(*planned, c.m, c.n, c.k);
+  std::vector<GridPart> best;
+
+  // the whole problem on another tile, or on the build of the planned one
+  const Build &whole = fastest(c.m, c.n, c.k);
+  if ((&whole != planned || !is_build(c, whole)) && grid_us(whole, c.m, c.n, c.k) < best_us) {
+    best_us = grid_us(whole, c.m, c.n, c.k);
+    best = {GridPart{on_build(c, whole, c.m, c.n)}};
+  }
+  // the rows, or columns, of whole rounds as planned and the rest on the
+  // tile that is fastest for it
+  const int64_t full = tiles / kCus * kCus;
+  for (const bool rows : {true, false}) {
+    const int64_t per_line = rows ? tn : tm, block = rows ? c.block_m : c.block_n;
+    const int64_t cut = full / per_line * block; // rows or columns of the first part
+    if (cut == 0 || cut >= (rows ? c.m : c.n))
+      continue;
+    const int64_t m0 = rows ? cut : c.m, n0 = rows ? c.n : cut;
+    const int64_t m1 = rows ? c.m - cut : c.m, n1 = rows ? c.n : c.n - cut;
+    const Build &rest = fastest(m1, n1, c.k);
+    // 2 us for what a second launch leaves idle at its start and end
+    const double us = over_build(c, *planned) * grid_us(*planned, m0, n0, c.k) +
+                      grid_us(rest, m1, n1, c.k) + 2;
+    if (us >= best_us)
+      continue;
+    best_us = us;
+    tb_gemm_config first = c;
+    first.m = m0;
+    first.n = n0;
+    const int64_t programs = ceil_div(m0, c.block_m) * ceil_div(n0, c.block_n);
+    first.num_programs = persistent ? std::min(c.num_programs, programs) : programs;
+    best = {GridPart{first},
+            GridPart{on_build(c, rest, m1, n1), rows ? cut : 0, rows ? 0 : cut}};
+  }
+  return best;
+}
+
+} // namespace tbrt

@@ -1,0 +1,23 @@
+// How a planned problem is spread over the chip: the choice of builds and
+// sub-problems one launch of a plan runs.
+#pragma once
+
+#include "tb_gfx950.h"
+
+#include <cstdint>
+#include <vector>
+
+namespace tbrt {
+
+// A rectangle of C computed by one kernel launch: rows row0 .. row0+m-1 and
+// columns col0 .. col0+n-1 of the problem, on the configuration `cfg` (whose
+// m and n are the rectangle's).
+struct GridPart {
+  tb_gemm_config cfg;
+  int64_t row0 = 0, col0 = 0;
+};
+
+// The rectangles a planned configuration runs as. Empty: as planned.
+std::vector<GridPart> split_grid(const tb_gemm_config &c);
+
+} // namespace tbrt

@@ -77,8 +77,10 @@ Planned configFromModule(tb::Module &m, const std::string &gpuArch) {
 int bindPlanned(const Planned &p, tb_gemm_desc **out, const char *who) {
   if (int rc = tbrt::create_desc(p.config, out))
     return rc;
-  if (p.waits.empty())
+  if (p.waits.empty()) {
+    tbrt::choose_parts(*out);
     return 0;
+  }
   int64_t have[3];
   tbrt::desc_waits(*out, have);
   if (p.waits.size() != 3 || p.waits[0] != have[0] || p.waits[1] != have[1] ||
@@ -94,6 +96,7 @@ int bindPlanned(const Planned &p, tb_gemm_desc **out, const char *who) {
     *out = nullptr;
     return fail(msg);
   }
+  tbrt::choose_parts(*out);
   return 0;
 }
 

@@ -1,0 +1,76 @@
+// The rectangles a plan's launch runs (csrc/runtime/grid_split.h) tile C
+// exactly, on whole planned tiles, for random plans of every shape and order;
+// split-K plans and plans that keep fewer programs than CUs run as they are.
+#include "runtime/grid_split.h"
+
+#include <cstdio>
+#include <cstdlib>
+#include <random>
+
+#define CHECK(x)                                                                            \
+  do {                                                                                      \
+    if (!(x)) {                                                                             \
+      std::printf("FAILED: %s (%lld x %lld x %lld on %lld x %lld, mapping %d)\n", #x,      \
+                  (long long)c.m, (long long)c.n, (long long)c.k, (long long)c.block_m,     \
+                  (long long)c.block_n, c.mapping);                                         \
+      std::exit(1);                                                                         \
+    }                                                                                       \
+  } while (0)
+
+static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+int main() {
+  std::mt19937 rng(7);
+  const int blocks[] = {64, 128, 192, 256};
+  int whole = 0, cut = 0;
+  for (int i = 0; i < 20000; ++i) {
+    tb_gemm_config c{};
+    c.m = 1 + rng() % (1u << (4 + rng() % 13));
+    c.n = 8 * (1 + rng() % (1u << (1 + rng() % 13)));
+    c.k = 8 * (1 + rng() % 1000);
+    c.block_m = blocks[rng() % 4];
+    c.block_n = blocks[rng() % 4];
+    c.block_k = rng() % 2 ? 64 : 32;
+    c.num_waves = 1 << rng() % 4;
+    c.stages = 2 + rng() % 3;
+    c.mapping = rng() % 5;
+    c.group_m = 8;
+    c.split_k = c.mapping == TB_MAP_SPLIT_K ? 4 : 1;
+    const int64_t tiles = ceil_div(c.m, c.block_m) * ceil_div(c.n, c.block_n);
+    const bool persistent =
+        c.mapping == TB_MAP_PERSISTENT_TILE || c.mapping == TB_MAP_PERSISTENT_GROUPED;
+    c.num_programs = persistent ? std::min<int64_t>(tiles, 1 + rng() % 512) : tiles * c.split_k;
+    const std::vector<tbrt::GridPart> parts = tbrt::split_grid(c);
+    if (c.mapping == TB_MAP_SPLIT_K ||
+        (persistent && c.num_programs < 256))
+      CHECK(parts.empty());
+    CHECK(parts.size() <= 2);
+    int64_t area = 0;
+    for (const tbrt::GridPart &p : parts) {
+      CHECK(p.row0 % c.block_m == 0 && p.col0 % c.block_n == 0);
+      CHECK(p.cfg.m > 0 && p.cfg.n > 0 && p.row0 + p.cfg.m <= c.m && p.col0 + p.cfg.n <= c.n);
+      CHECK(p.cfg.k == c.k && p.cfg.split_k == 1 && p.cfg.n % 8 == 0);
+      const int64_t t = ceil_div(p.cfg.m, p.cfg.block_m) * ceil_div(p.cfg.n, p.cfg.block_n);
+      const bool pers = p.cfg.mapping == TB_MAP_PERSISTENT_TILE ||
+                        p.cfg.mapping == TB_MAP_PERSISTENT_GROUPED;
+      CHECK(pers ? p.cfg.num_programs <= t : p.cfg.num_programs == t);
+      area += p.cfg.m * p.cfg.n;
+    }
+    if (parts.size() == 2) { // side by side: the second starts where the first ends
+      const tbrt::GridPart &a = parts[0], &b = parts[1];
+      CHECK(a.row0 == 0 && a.col0 == 0);
+      CHECK((b.row0 == a.cfg.m && b.col0 == 0 && b.cfg.n == c.n) ||
+            (b.col0 == a.cfg.n && b.row0 == 0 && b.cfg.m == c.m));
+      CHECK(a.cfg.block_m == c.block_m && a.cfg.mapping == c.mapping);
+    }
+    CHECK(parts.empty() || area == c.m * c.n);
+    whole += parts.size() == 1;
+    cut += parts.size() == 2;
+  }
+  if (whole < 1000 || cut < 10) {
+    std::printf("FAILED: only %d whole and %d cut problems\n", whole, cut);
+    return 1;
+  }
+  std::printf("ok: %d whole, %d cut\n", whole, cut);
+  return 0;
+}

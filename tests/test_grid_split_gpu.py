@@ -1,0 +1,65 @@
+"""The launches of a plan whose grid leaves CUs idle, or a last round nearly
+empty, run on other tiles or as two rectangles of C. Each result is compared
+bit for bit with the planned kernel itself (a descriptor made from the plan's
+configuration runs exactly that): a whole problem on a finer tile, on a
+coarser one, rows and columns cut off as a second rectangle, ragged in M, N
+and K, with a bias row, an f32 C and persistent order; padding past the
+result is not written."""
+import pytest
+import torch
+
+import mini_triton_nvgpu_v1_amd as tb
+from mini_triton_nvgpu_v1_amd import configs
+
+pytestmark = pytest.mark.gpu
+
+BIG, MID, SMALL = (256, 256, 64), (128, 128, 64), (64, 64, 64)
+# (M, N, K, block, stages, options)
+CASES = [
+    (1, 8, 8, MID, 3, {}),                        # one element row, K below a k-tile
+    (129, 136, 72, MID, 2, {"bias": "f16", "activation": "silu"}),
+    (1000, 1496, 712, BIG, 2, {"bias": "f32", "clamp_min": -0.5, "clamp_max": 0.5}),
+    (900, 1032, 1032, MID, 2, {}),                # 2-stage plan with a long K
+    (2048, 2056, 200, SMALL, 2, {}),              # a coarser tile
+    (4104, 4096, 520, BIG, 2, {"bias": "f16"}),   # 8 rows past a whole round
+    (512, 40000, 264, BIG, 2, {"bias": "f32"}),   # columns cut off
+    (4200, 4200, 328, BIG, 2, {"persistent": True, "num_ctas": 256}),
+    (4200, 4200, 328, BIG, 2, {"c_f32": True}),
+    (700, 1504, 2048, BIG, 2, {"c_f32": True}),
+]
+
+
+@pytest.mark.parametrize("M,N,K,block,stages,options", CASES,
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else None)
+def test_matches_planned_kernel(M, N, K, block, stages, options, device):
+    print(f"grid split {M}x{N}x{K} {block} {options}", flush=True)
+    w = configs.Workload("w", M, N, K, 0, configs.NORMAL, block, num_waves=4, stages=stages,
+                         exact_tile=False, **options)
+    plan = tb.plan_from_mlir(w.mlir())
+    exact = tb.GemmDesc.from_config(plan.config)
+    assert exact.kernel_name == plan.kernel_name
+    g = torch.Generator(device=device).manual_seed(M + N + K)
+    a = torch.randn(M, K, generator=g, device=device).half()
+    b = (torch.randn(K, N, generator=g, device=device) / K ** 0.5).half()
+    bias = None
+    if w.bias:
+        bias = torch.randn(N, generator=g, device=device,
+                           dtype=torch.float16 if w.bias == "f16" else torch.float32)
+    got = []
+    for desc in (plan, exact):
+        # C in the middle of a larger buffer whose ends must stay as they are
+        buf = torch.full((M * N + 512,), 3.0, device=device,
+                         dtype=torch.float32 if w.c_f32 else torch.float16)
+        c = buf[256:256 + M * N].view(M, N)
+        desc.launch(a, b, c, bias=bias)
+        assert (buf[:256] == 3).all() and (buf[256 + M * N:] == 3).all()
+        got.append(c)
+    if w.c_f32:
+        # the prior C is added before or after the products: one rounding of
+        # each running sum apart
+        mag = a.float().abs() @ b.float().abs() + 3
+        assert ((got[0] - got[1]).abs() <= (K + 2) * 2.0 ** -23 * mag).all()
+        ref = a.double() @ b.double() + 3
+        assert ((got[0] - ref).abs() <= (K + 2) * 2.0 ** -24 * mag).all()
+    else:
+        assert torch.equal(got[0], got[1])
