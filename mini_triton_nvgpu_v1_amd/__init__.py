@@ -201,11 +201,44 @@ def _check_operand(x, role: str, dtypes: tuple, rows: int, cols: int, ld: int,
                           f"{tuple(x.shape)}, strides {tuple(x.stride())})")
 
 
+_raw_stream = None
+
+
+def _current_stream(dev: int) -> int:
+    """The handle of torch's current stream on GPU `dev`: torch's raw accessor
+    where it has one (0.1 us; building the Stream object takes 1.1)."""
+    global _raw_stream
+    if _raw_stream is None:
+        import torch
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+            lambda d: torch.cuda.current_stream(d).cuda_stream)
+    return _raw_stream(dev)
+
+
+class _Expected:
+    """What a descriptor's operands are checked against. A descriptor is
+    immutable, so this is read from the C ABI once per descriptor."""
+    __slots__ = ("torch", "dtype_c", "dtype_bias", "shapes", "n", "plain", "ws_bytes")
+
+    def __init__(self, cf: GemmConfig, ws_bytes: int):
+        import torch
+        self.torch = torch
+        self.dtype_c = torch.float16 if cf.c_dtype == DTYPE_F16 else torch.float32
+        self.dtype_bias = {EPI_BIAS_NONE: None, EPI_BIAS_F16: torch.float16,
+                           EPI_BIAS_F32: torch.float32}[cf.epi_bias]
+        self.shapes = ((cf.m, cf.k), (cf.k, cf.n), (cf.m, cf.n))
+        self.n = cf.n
+        # whole matrices: every leading dimension is its row length
+        self.plain = (cf.lda, cf.ldb, cf.ldc) == (cf.k, cf.n, cf.n)
+        self.ws_bytes = ws_bytes
+
+
 class GemmDesc:
     """Owning handle of a ``tb_gemm_desc``."""
 
     def __init__(self, handle: int):
         self._h = ctypes.c_void_p(handle)
+        self._expected = None
 
     @classmethod
     def from_config(cls, cfg: GemmConfig | None = None, **fields) -> "GemmDesc":
@@ -268,6 +301,53 @@ class GemmDesc:
         if len(devs) > 1:
             raise TbError(f"operands are on different devices: {sorted(map(str, devs))}")
 
+    def _plain_operands(self, a, b, c, workspace, bias) -> int | None:
+        """The device index when the operands are the common case, whole
+        contiguous matrices (and a bias vector and workspace) in plain tensors
+        on one GPU: then check_operands has nothing to refuse. None: anything
+        else, which check_operands looks at. A call's checks cost as much as
+        its launch, and these read each tensor's few fields once (64x64x32:
+        12.3 us per launch() with check_operands, 5.1 this way)."""
+        e = self._expected
+        if e is None:
+            if not _is_tensor(a):
+                return None
+            e = self._expected = _Expected(self.config, self.workspace_bytes)
+        if not e.plain:
+            return None
+        tensor, half = e.torch.Tensor, e.torch.float16
+        if not (type(a) is tensor and type(b) is tensor and type(c) is tensor):
+            return None
+        sa, sb, sc = e.shapes
+        if not (a.dtype is half and b.dtype is half and c.dtype is e.dtype_c
+                and a.shape == sa and b.shape == sb and c.shape == sc
+                and a.is_contiguous() and b.is_contiguous() and c.is_contiguous()):
+            return None
+        dev = a.get_device()
+        if dev < 0 or b.get_device() != dev or c.get_device() != dev:
+            return None
+        # a storage may have been shrunk under its tensor
+        for x in (a, b, c):
+            if ((x.storage_offset() + x.numel()) * x.element_size()
+                    > x.untyped_storage().nbytes()):
+                return None
+        if bias is not None:
+            if not (type(bias) is tensor and bias.dtype is e.dtype_bias
+                    and bias.shape == (e.n,) and bias.is_contiguous()
+                    and bias.get_device() == dev
+                    and (bias.storage_offset() + e.n) * bias.element_size()
+                    <= bias.untyped_storage().nbytes()):
+                return None
+        if workspace is not None:
+            if not (type(workspace) is tensor and workspace.dim() == 1
+                    and workspace.is_contiguous() and workspace.get_device() == dev):
+                return None
+            held = (workspace.untyped_storage().nbytes()
+                    - workspace.storage_offset() * workspace.element_size())
+            if held < e.ws_bytes:
+                return None
+        return dev
+
     @staticmethod
     def _default_stream(stream, *xs):
         """An explicit stream wins; else torch's current stream of the
@@ -281,30 +361,40 @@ class GemmDesc:
                 return torch.cuda.current_stream(x.device).cuda_stream
         return None
 
+    def _checked_stream(self, stream, a, b, c, workspace, bias) -> int | None:
+        """Check the operands; the stream handle of the launch."""
+        dev = self._plain_operands(a, b, c, workspace, bias)
+        if dev is None:
+            self.check_operands(a, b, c, workspace, bias)
+            return self._default_stream(stream, a, b, c)
+        if stream is None:
+            return _current_stream(dev)
+        return _stream_handle(stream)
+
     def launch(self, a, b, c, workspace=None, stream=None, bias=None) -> None:
         """Enqueue C = A*B (or C += A*B), then the config's fused epilogue
         steps, for device tensors/addresses. ``bias`` (N values) is required
         exactly when the config adds one. Tensors are checked against the
         descriptor (check_operands); ``stream`` defaults to torch's current
         stream of the tensors' device."""
-        self.check_operands(a, b, c, workspace, bias)
-        st = self._default_stream(stream, a, b, c)
+        st = self._checked_stream(stream, a, b, c, workspace, bias)
         if bias is None:
-            _check(lib().tb_gemm_launch(self._h, _ptr(a), _ptr(b), _ptr(c),
-                                        _ptr(workspace), st))
+            rc = _lib.tb_gemm_launch(self._h, _ptr(a), _ptr(b), _ptr(c), _ptr(workspace), st)
         else:
-            _check(lib().tb_gemm_launch_ex(self._h, _ptr(a), _ptr(b), _ptr(c),
-                                           _ptr(bias), _ptr(workspace), st))
+            rc = _lib.tb_gemm_launch_ex(self._h, _ptr(a), _ptr(b), _ptr(c), _ptr(bias),
+                                        _ptr(workspace), st)
+        if rc:
+            _check(rc)
 
     def launch_noalloc(self, a, b, c, stream=None, bias=None) -> None:
         """Like launch, with no workspace argument: a split-K descriptor's
         partials go to the library's static per-GPU scratch
         (NOALLOC_SCRATCH_BYTES), and nothing is allocated. Calls that overlap
         on one GPU share that scratch and race."""
-        self.check_operands(a, b, c, None, bias)
-        st = self._default_stream(stream, a, b, c)
-        _check(lib().tb_gemm_launch_noalloc(self._h, _ptr(a), _ptr(b), _ptr(c),
-                                            _ptr(bias), st))
+        st = self._checked_stream(stream, a, b, c, None, bias)
+        rc = _lib.tb_gemm_launch_noalloc(self._h, _ptr(a), _ptr(b), _ptr(c), _ptr(bias), st)
+        if rc:
+            _check(rc)
 
     def bind(self, a, b, c, workspace=None, stream=None, bias=None):
         """A zero-argument launcher for repeated launches on the same buffers
