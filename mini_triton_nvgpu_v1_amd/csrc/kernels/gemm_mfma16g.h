@@ -611,10 +611,8 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_mfma16g(GemmParams p) {
   __shared__ u32x4 lds[T::LDS_BYTES / 16];
   const bool persistent =
       p.mapping == kMapPersistent || p.mapping == kMapPersistentGrouped;
-  int prog = blockIdx.x;
   const int nprog = gridDim.x;
-  if (p.xcds > 1 && (nprog % p.xcds) == 0)
-    prog = (prog % p.xcds) * (nprog / p.xcds) + prog / p.xcds;
+  const int prog = program_of_block(blockIdx.x, nprog, p.xcds);
   for (int work = prog; work < p.total_work;
        work += (persistent ? nprog : p.total_work)) {
     int tile_m, tile_n, part;
