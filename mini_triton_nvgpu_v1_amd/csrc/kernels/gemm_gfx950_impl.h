@@ -105,20 +105,6 @@ __device__ __forceinline__ GemmParams params_fresh() {
   return r;
 }
 
-// First statement of each variant of a dispatched epilogue: an empty asm
-// that differs per (activation, clamp), so the variants no longer begin with
-// the same code, and a scheduling barrier that keeps the variant's own code
-// below it. Otherwise the compiler hoists their common start (the
-// accumulator reads of every element) above the dispatch, holding the whole
-// tile in VGPRs at once (the fused 16x16x32 build spilled).
-template <int ACT, bool CLAMP>
-__device__ __forceinline__ void epi_variant_fence() {
-  asm volatile("; fused epilogue variant %0 %1" ::"i"(ACT), "i"(CLAMP ? 1 : 0));
-  __builtin_amdgcn_sched_barrier(0); // nothing scheduled above it
-}
-
-
-
 // f(std::integral_constant<int, i>{}) for i = 0 .. N-1, in order.
 template <class F, int... I>
 __device__ __forceinline__ void static_for_seq(F &&f, std::integer_sequence<int, I...>) {
@@ -147,19 +133,42 @@ __device__ __forceinline__ void acc_read_fence(f32x4 (&acc)[TI][TJ]) {
       asm volatile("" : "+a"(acc[i][j]));
 }
 
-// Runs block(i, act, clamp) for the epilogue's 16-row blocks i = 0 .. NB-1,
-// with EPI the activation and clamp of the launch dispatched once per block
-// (a block's code is specialised to them); without, the plain block.
-// Dispatched per block rather than once for the whole tile, a variant reads
-// only one block's accumulators, whatever the compiler hoists above it.
-template <int NB, bool EPI, class F>
-__device__ __forceinline__ void epi_for_blocks(const GemmParams &pe, F &&block) {
-  static_for<NB>([&](auto i_c) {
-    if constexpr (EPI)
-      epi_dispatch(pe.epi_act, pe.epi_clamp, [&](auto a, auto c) { block(i_c, a, c); });
-    else
-      block(i_c, std::integral_constant<int, 0>{}, std::integral_constant<bool, false>{});
-  });
+// Runs block(i, act, clamp) for the epilogue's 16-row blocks i = 0 .. NB-1
+// of the accumulators; with EPI, in the variant specialised to the launch's
+// activation and clamp. ONCE dispatches it once for the tile: a lone wave
+// runs this code once, straight through, and every jump in it waits for code
+// the instruction cache does not hold (4096^3 with bias and GELU: 111.4 us
+// with the dispatch in front of each of the 8 blocks at 97.0 plain, 99.1 at
+// 93.5 dispatched once; 103.9 at 99.6 with no dispatch at all). C += A*B
+// dispatches per block: the prior C's blocks it holds ahead leave no room for
+// the registers a whole variant takes (it spilled). Each block's accumulators
+// pass through an asm (no instruction) that differs per (activation, clamp):
+// the variants then share no accumulator read that the compiler could hoist
+// above the dispatch, where it would hold the whole tile in VGPRs at once.
+template <bool EPI, bool ONCE, int NB, int TJ, class F>
+__device__ __forceinline__ void epi_for_blocks(const GemmParams &pe, f32x4 (&acc)[NB][TJ],
+                                               F &&block) {
+  auto variant = [&](auto i_c, auto act_c, auto clamp_c) {
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+      asm volatile("; fused epilogue variant %1 %2"
+                   : "+a"(acc[decltype(i_c)::value][j])
+                   : "i"(decltype(act_c)::value), "i"(decltype(clamp_c)::value ? 1 : 0));
+    __builtin_amdgcn_sched_barrier(0); // nothing scheduled above it
+    block(i_c, act_c, clamp_c);
+  };
+  if constexpr (EPI && ONCE)
+    epi_dispatch(pe.epi_act, pe.epi_clamp, [&](auto act_c, auto clamp_c) {
+      static_for<NB>([&](auto i_c) { variant(i_c, act_c, clamp_c); });
+    });
+  else
+    static_for<NB>([&](auto i_c) {
+      if constexpr (EPI)
+        epi_dispatch(pe.epi_act, pe.epi_clamp,
+                     [&](auto act_c, auto clamp_c) { variant(i_c, act_c, clamp_c); });
+      else
+        block(i_c, std::integral_constant<int, 0>{}, std::integral_constant<bool, false>{});
+    });
 }
 
 // Raw buffer descriptor as four dwords for inline asm operands ("s"): the
@@ -803,7 +812,6 @@ __device__ __forceinline__ void mfma16_tile(const GemmParams &p, int m0, int n0,
       constexpr int i = decltype(i_c)::value;
       constexpr int ACT = decltype(act_c)::value;
       constexpr bool CLAMP = decltype(clamp_c)::value;
-      epi_variant_fence<ACT, CLAMP>();
       const int r = 16 * i + (el & 15);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -842,7 +850,7 @@ __device__ __forceinline__ void mfma16_tile(const GemmParams &p, int m0, int n0,
       }
       __builtin_amdgcn_sched_barrier(0);
     };
-    epi_for_blocks<8, EPI>(pe, block);
+    epi_for_blocks<EPI, OUT != kOutF32Accum>(pe, acc, block);
   } else {
     // f32 C through LDS, one 16-row block of the wave tile at a time. Lane l
     // holds row 16i + l%16, columns 16j + 4(l/16) .. +3 of block i (16 bytes
@@ -889,7 +897,6 @@ __device__ __forceinline__ void mfma16_tile(const GemmParams &p, int m0, int n0,
       constexpr int i = decltype(i_c)::value;
       constexpr int ACT = decltype(act_c)::value;
       constexpr bool CLAMP = decltype(clamp_c)::value;
-      epi_variant_fence<ACT, CLAMP>();
       TBK_LDS char *blk = wl + (i & 3) * 8192;
       const int r = el & 15, g = el >> 4;
 #pragma unroll
@@ -921,7 +928,7 @@ __device__ __forceinline__ void mfma16_tile(const GemmParams &p, int m0, int n0,
         load_old(i + PF);
       __builtin_amdgcn_sched_barrier(0);
     };
-    epi_for_blocks<8, EPI>(pe, block);
+    epi_for_blocks<EPI, OUT != kOutF32Accum>(pe, acc, block);
   }
 }
 

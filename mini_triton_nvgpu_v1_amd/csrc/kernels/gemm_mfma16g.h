@@ -495,7 +495,6 @@ __device__ __forceinline__ void mfma16g_tile(const GemmParams &p, int m0, int n0
       constexpr int i = decltype(i_c)::value;
       constexpr int ACT = decltype(act_c)::value;
       constexpr bool CLAMP = decltype(clamp_c)::value;
-      epi_variant_fence<ACT, CLAMP>();
 #pragma unroll
       for (int j = 0; j < TJ; ++j) {
         float x[4];
@@ -532,7 +531,7 @@ __device__ __forceinline__ void mfma16g_tile(const GemmParams &p, int m0, int n0
       }
       __builtin_amdgcn_sched_barrier(0);
     };
-    epi_for_blocks<TI, EPI>(pe, block);
+    epi_for_blocks<EPI, OUT != kOutF32Accum>(pe, acc, block);
   } else {
     // f32: lane l holds row r = l % 16 of block i, columns 16 j + 4 (l / 16)
     // .. +3, 16 bytes at chunk 4 j + l / 16, placed at chunk ^ ((r /
@@ -572,7 +571,6 @@ __device__ __forceinline__ void mfma16g_tile(const GemmParams &p, int m0, int n0
       constexpr int i = decltype(i_c)::value;
       constexpr int ACT = decltype(act_c)::value;
       constexpr bool CLAMP = decltype(clamp_c)::value;
-      epi_variant_fence<ACT, CLAMP>();
 #pragma unroll
       for (int j = 0; j < TJ; ++j) {
         *(TBK_LDS f32x4 *)(wl + r * T::E32_ROWB + (((4 * j + gg) ^ xr) * 16)) = acc[i][j];
@@ -600,7 +598,7 @@ __device__ __forceinline__ void mfma16g_tile(const GemmParams &p, int m0, int n0
         load_old(i + PF);
       __builtin_amdgcn_sched_barrier(0);
     };
-    epi_for_blocks<TI, EPI>(pe, block);
+    epi_for_blocks<EPI, OUT != kOutF32Accum>(pe, acc, block);
   }
 }
 
