@@ -1203,10 +1203,26 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_kernel(GemmParams p) {
         if (T::load_off(l) < T::AFTER)
           issue_load(kt0 + STAGES - 1, STAGES - 1, l);
     } else {
+      // only the k-tiles there are: a short K would otherwise wait for loads
+      // of zeros
 #pragma unroll
       for (int st = 0; st < STAGES; ++st)
-        issue_tile(kt0 + st, st);
+        if (st == 0 || st < nk)
+          issue_tile(kt0 + st, st);
     }
+    // burst schedule: the wait for a k-tile behind which `tiles` more are in
+    // flight, and EXTRA other loads
+    auto wait_tiles = [&](int tiles, auto extra_c) {
+      constexpr int EXTRA = decltype(extra_c)::value;
+      if (tiles >= STAGES - 1)
+        wait_vmcnt<(STAGES - 1) * LPT + EXTRA>();
+      else if (STAGES > 2 && tiles == STAGES - 2)
+        wait_vmcnt<(STAGES - 2) * LPT + EXTRA>();
+      else if (STAGES > 3 && tiles == STAGES - 3)
+        wait_vmcnt<(STAGES > 3 ? STAGES - 3 : 0) * LPT + EXTRA>();
+      else
+        wait_vmcnt<EXTRA>();
+    };
     if constexpr (C_ROWS_EARLY) {
       const __amdgpu_buffer_rsrc_t rc =
           make_rsrc(rows_at(p.C, m0, p.ldc, 4), rows_bytes(m0, p.M, p.ldc, 4));
@@ -1225,9 +1241,14 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_kernel(GemmParams p) {
         }
       // the prior C loads are the youngest: k-tile 0 has landed once at most
       // VM_PROLOGUE of the A/B loads and all of them are outstanding
-      wait_vmcnt<T::VM_PROLOGUE + TM * NLD32>();
-    } else {
+      if constexpr (T::SLOTTED)
+        wait_vmcnt<T::VM_PROLOGUE + TM * NLD32>();
+      else
+        wait_tiles(nk - 1, std::integral_constant<int, TM * NLD32>{});
+    } else if constexpr (T::SLOTTED) {
       wait_vmcnt<T::VM_PROLOGUE>();
+    } else {
+      wait_tiles(nk - 1, std::integral_constant<int, 0>{});
     }
     __syncthreads();
     read_frags(0, 0, 0);
@@ -1285,33 +1306,56 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_kernel(GemmParams p) {
         sp = s;
         s = s_next;
       }
-    } else
-    for (int it = 0; it < nk; ++it) {
-      const int s_next = s + 1 == STAGES ? 0 : s + 1;
+    } else {
+      // Burst schedule. The k-tiles whose refill exists run the loop; the
+      // last STAGES ones run a copy that waits for, reads and loads only
+      // what there is (K up to a few k-tiles, where lookahead loads of zeros
+      // and the barrier after the last k-tile were 0.3 us of a 3 us kernel:
+      // 448x288x64 on 64x64x64, f32 C += A*B: 3.22 -> 2.93 us; the tail's
+      // branches in the loop itself cost 7% at K = 4096). After a barrier
+      // the refill goes out before the fragment reads (1024^2 x 4096, 64x64x64
+      // in 3 stages: 21.3 -> 20.1; 64x128x64 on 1x4 waves: 26.8 -> 25.7; in 2
+      // stages 31.2 -> 31.1).
+      auto ktile = [&](int it, auto tail_c) {
+        constexpr bool TAIL = decltype(tail_c)::value;
+        const int s_next = s + 1 == STAGES ? 0 : s + 1;
 #pragma unroll
-      for (int ks = 0; ks < KSTEPS; ++ks) {
-        const int cur = ks & 1;
-        if (ks + 1 < KSTEPS) {
-          read_frags(cur ^ 1, s, ks + 1);
-          mfma_range(cur, 0, NMFMA);
-          if (ks == 0)
+        for (int ks = 0; ks < KSTEPS; ++ks) {
+          const int cur = ks & 1;
+          if (ks + 1 < KSTEPS) {
+            read_frags(cur ^ 1, s, ks + 1);
+            mfma_range(cur, 0, NMFMA);
             sched_step<NMFMA, TM + 2 * TN, 0>();
-          else
-            sched_step<NMFMA, TM + 2 * TN, 0>();
-          __builtin_amdgcn_sched_barrier(0); // k steps do not mix
-        } else {
-          mfma_range(cur, 0, NMFMA / 2);
-          __builtin_amdgcn_sched_barrier(0);
-          wait_vmcnt<T::VM_LOOP>();
-          __syncthreads();
-          read_frags(cur ^ 1, s_next, 0);
-          issue_tile(kt0 + it + STAGES, s);
-          mfma_range(cur, NMFMA / 2, NMFMA);
-          sched_step<NMFMA - NMFMA / 2, TM + 2 * TN, 0>();
-          __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_sched_barrier(0); // k steps do not mix
+          } else {
+            mfma_range(cur, 0, NMFMA / 2);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (!TAIL) {
+              wait_vmcnt<T::VM_LOOP>();
+              __syncthreads();
+              // the refill first: it is what the next barriers wait for
+              issue_tile(kt0 + it + STAGES, s);
+              __builtin_amdgcn_sched_barrier(0);
+              read_frags(cur ^ 1, s_next, 0);
+            } else if (it + 1 < nk) {
+              wait_tiles(nk - 2 - it, std::integral_constant<int, 0>{});
+              __syncthreads();
+              read_frags(cur ^ 1, s_next, 0);
+            }
+            mfma_range(cur, NMFMA / 2, NMFMA);
+            if constexpr (!TAIL)
+              sched_step<NMFMA - NMFMA / 2, TM + 2 * TN, 0>();
+            __builtin_amdgcn_sched_barrier(0);
+          }
         }
-      }
-      s = s_next;
+        s = s_next;
+      };
+      int it = 0;
+      for (; it + STAGES < nk; ++it)
+        ktile(it, std::integral_constant<bool, false>{});
+#pragma nounroll
+      for (; it < nk; ++it)
+        ktile(it, std::integral_constant<bool, true>{});
     }
 
     // Drain the (out-of-range, zero) loads still in flight into LDS so none
