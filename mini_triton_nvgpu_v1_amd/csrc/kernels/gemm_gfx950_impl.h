@@ -1575,7 +1575,8 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_kernel(GemmParams p) {
             // splits on one line at a time) measured 1 us slower, all splits
             // of a tile on one XCD 0.3-2 us slower.
             constexpr int NA = BR * T::WTN / 64; // dwords per lane per pass
-#pragma unroll
+            // 8 at a time: unrolled whole, 8 waves of 64x128 ran out of registers
+#pragma unroll 8
             for (int t = 0; t < NA; ++t) {
               const int r = (t * 64 + lane) / T::WTN; // row of the pass
               const int c = (t * 64 + lane) % T::WTN; // column of the wave tile
