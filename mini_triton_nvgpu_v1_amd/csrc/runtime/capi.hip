@@ -320,7 +320,8 @@ int launch_impl(const tb_gemm_desc *d, const void *a, const void *b, void *c,
   if (d->parts.empty())
     return launch_kernels(d, a, b, c, bias, workspace, s);
   // a part starts at whole tiles and every leading dimension is a multiple
-  // of 8 elements, so the offset operands keep the alignment checked above
+  // of 8 elements, so the offset operands keep the alignment checked above;
+  // a split-K plan's one part has its workspace
   const tb_gemm_config &cf = d->cfg;
   const int64_t c_size = cf.c_dtype == TB_DTYPE_F16 ? 2 : 4;
   const int64_t bias_size = cf.epi_bias == TB_EPI_BIAS_F16 ? 2 : 4;
@@ -330,7 +331,7 @@ int launch_impl(const tb_gemm_desc *d, const void *a, const void *b, void *c,
             part.desc.get(), static_cast<const char *>(a) + r0 * cf.lda * 2,
             static_cast<const char *>(b) + c0 * 2,
             static_cast<char *>(c) + (r0 * cf.ldc + c0) * c_size,
-            bias ? static_cast<const char *>(bias) + c0 * bias_size : nullptr, nullptr, s))
+            bias ? static_cast<const char *>(bias) + c0 * bias_size : nullptr, workspace, s))
       return rc;
   }
   return 0;

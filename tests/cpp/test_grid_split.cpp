@@ -1,6 +1,7 @@
 // The rectangles a plan's launch runs (csrc/runtime/grid_split.h) tile C
 // exactly, on whole planned tiles, for random plans of every shape and order;
-// split-K plans and plans that keep fewer programs than CUs run as they are.
+// split-K plans keep their splits, and persistent plans of fewer programs than
+// CUs run as they are.
 #include "runtime/grid_split.h"
 
 #include <cstdio>
@@ -41,9 +42,17 @@ int main() {
         c.mapping == TB_MAP_PERSISTENT_TILE || c.mapping == TB_MAP_PERSISTENT_GROUPED;
     c.num_programs = persistent ? std::min<int64_t>(tiles, 1 + rng() % 512) : tiles * c.split_k;
     const std::vector<tbrt::GridPart> parts = tbrt::split_grid(c);
-    if (c.mapping == TB_MAP_SPLIT_K ||
-        (persistent && c.num_programs < 256))
+    if (persistent && c.num_programs < 256)
       CHECK(parts.empty());
+    if (c.mapping == TB_MAP_SPLIT_K) { // as planned but for the stages
+      for (const tbrt::GridPart &p : parts) {
+        CHECK(p.row0 == 0 && p.col0 == 0 && c.stages == 2 && p.cfg.stages == 3);
+        CHECK(p.cfg.m == c.m && p.cfg.n == c.n && p.cfg.split_k == c.split_k &&
+              p.cfg.reduction == c.reduction && p.cfg.num_programs == c.num_programs);
+      }
+      CHECK(parts.size() <= 1);
+      continue;
+    }
     CHECK(parts.size() <= 2);
     int64_t area = 0;
     for (const tbrt::GridPart &p : parts) {

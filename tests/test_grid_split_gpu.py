@@ -26,6 +26,7 @@ CASES = [
     (4200, 4200, 328, BIG, 2, {"persistent": True, "num_ctas": 256}),
     (4200, 4200, 328, BIG, 2, {"c_f32": True}),
     (700, 1504, 2048, BIG, 2, {"c_f32": True}),
+    (300, 520, 5000, MID, 2, {"split_k": 4, "bias": "f16"}),  # 3 stages for 2
 ]
 
 
@@ -51,7 +52,8 @@ def test_matches_planned_kernel(M, N, K, block, stages, options, device):
         buf = torch.full((M * N + 512,), 3.0, device=device,
                          dtype=torch.float32 if w.c_f32 else torch.float16)
         c = buf[256:256 + M * N].view(M, N)
-        desc.launch(a, b, c, bias=bias)
+        ws = torch.empty(max(desc.workspace_bytes, 16), dtype=torch.uint8, device=device)
+        desc.launch(a, b, c, ws, bias=bias)
         assert (buf[:256] == 3).all() and (buf[256 + M * N:] == 3).all()
         got.append(c)
     if w.c_f32:
