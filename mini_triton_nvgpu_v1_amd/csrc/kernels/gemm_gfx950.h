@@ -223,6 +223,9 @@ struct KernelEntry {
 const KernelEntry *find_kernel(const KernelKey &k);
 int kernel_count();
 const KernelEntry *kernel_at(int i);
+// The split-K build of a 16x16x32 tile (not in the registry: no plan names
+// it), or null.
+const KernelEntry *find_split_kernel(const KernelKey &k);
 
 // C = epilogue([C +] sum_{p < split_k} ws[p]) in fixed p order, cast to C's type.
 hipError_t launch_reduce_ex(const float *ws, void *C, int M, int N, int ldc,

@@ -203,20 +203,35 @@ struct Mfma16GTile {
   static_assert(tables_cover(), "per-slot tables hold every read and load");
 };
 
-template <int BM, int BN, int BK, int WGM, int WGN, int STAGES, int OUT, bool EPI>
-__device__ __forceinline__ void mfma16g_tile(const GemmParams &p, int m0, int n0, u32x4 *lds) {
+// SPLIT: split `part` of a split-K problem, its partial sums stored to plane
+// `part` of the workspace (kOutF32Partial) or added to C (kOutF32Atomic). The
+// split's k range is a GEMM of its own on A and B moved to its first k.
+template <int BM, int BN, int BK, int WGM, int WGN, int STAGES, int OUT, bool EPI,
+          bool SPLIT = false>
+__device__ __forceinline__ void mfma16g_tile(const GemmParams &p, int m0, int n0, u32x4 *lds,
+                                             int part = 0) {
   using T = Mfma16GTile<BM, BN, BK, WGM, WGN, STAGES>;
   constexpr int TI = T::TI, TJ = T::TJ, KS = T::KS, NM = T::NM, NR = T::NR, BQ = T::BQ;
   constexpr int LA = T::LA, LPT = T::LPT, U = T::U;
-  static_assert(OUT == kOutF16 || OUT == kOutF32Partial || OUT == kOutF32Accum,
-                "no atomic or split-K output on the 16x16x32 loop");
+  static_assert(SPLIT ? (OUT == kOutF32Partial || OUT == kOutF32Atomic) && !EPI
+                      : OUT == kOutF16 || OUT == kOutF32Partial || OUT == kOutF32Accum,
+                "output modes of the 16x16x32 loop");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(TBK_LDS void *)lds;
-  const int nk = (p.K + BK - 1) / BK;
-  const int kfull = p.K / BK;
-  const int krem = p.K - kfull * BK; // k values of the partial k-tile
+  int k0 = 0, klen = p.K; // the k range
+  if constexpr (SPLIT) {
+    // LowerPipelineToNVGPU.cpp:331-356 (contiguous k-tile range per split)
+    const int base = p.tiles_k / p.split_k, extra = p.tiles_k % p.split_k;
+    k0 = (part * base + (part < extra ? part : extra)) * BK;
+    const int tiles = base + (part < extra ? 1 : 0);
+    klen = k0 + tiles * BK < p.K ? tiles * BK : p.K - k0;
+    klen = klen > 0 ? klen : 0; // fewer k-tiles than splits
+  }
+  const int nk = (klen + BK - 1) / BK;
+  const int kfull = klen / BK;
+  const int krem = klen - kfull * BK; // k values of the partial k-tile
 
   // ---- direct-load geometry ----------------------------------------------
   // Round R of thread t = 64 wave + lane fills 16 bytes at R * NT * 16 + 16 t
@@ -225,11 +240,14 @@ __device__ __forceinline__ void mfma16g_tile(const GemmParams &p, int m0, int n0
   const int t = wave * 64 + lane;
   const int a_r0 = t / T::CPRA, a_pc = t % T::CPRA;
   const int b_r0 = t / T::CPRB, b_pc = t % T::CPRB;
-  const void *a_tile = rows_at(p.A, m0, p.lda, 2); // A's window starts at row m0
+  // A's window starts at row m0 (and the split's first k)
+  const void *a_tile =
+      static_cast<const char *>(rows_at(p.A, m0, p.lda, 2)) + (size_t)k0 * 2u;
+  const void *b_mat = rows_at(p.B, k0, p.ldb, 2);
   // A rows past M fall outside the window's records (it ends at row M) and
   // load zeros; B columns past N get the offset kOob
-  const uint32_t a_bytes = rows_bytes(m0, p.M, p.lda, 2);
-  const uint32_t b_bytes = (uint32_t)p.K * (uint32_t)p.ldb * 2u;
+  const uint32_t a_bytes = rows_bytes(m0, p.M, p.lda, 2) - (uint32_t)k0 * 2u;
+  const uint32_t b_bytes = (uint32_t)klen * (uint32_t)p.ldb * 2u;
   // per swizzle phase (round mod PA / PB): the vector offset; for the A
   // rounds also the same offset with the partial k-tile's mask (chunks at
   // or past K load from kOob)
@@ -266,7 +284,7 @@ __device__ __forceinline__ void mfma16g_tile(const GemmParams &p, int m0, int n0
   };
   // descriptors of k-tile kt: zero records past the last k-tile
   auto rsrc_a = [&](int kt) { return rsrc_dwords(a_tile, kt < nk ? a_bytes : 0u); };
-  auto rsrc_b = [&](int kt) { return rsrc_dwords(p.B, kt < nk ? b_bytes : 0u); };
+  auto rsrc_b = [&](int kt) { return rsrc_dwords(b_mat, kt < nk ? b_bytes : 0u); };
 
   // ---- fragment reads ----------------------------------------------------
   const int g = lane >> 4, ta = (lane >> 2) & 3, tb = lane & 3;
@@ -543,12 +561,17 @@ __device__ __forceinline__ void mfma16g_tile(const GemmParams &p, int m0, int n0
     constexpr int PF = OUT == kOutF32Accum ? cmin(TI, EPI ? 2 : 4) : 1;
     const int q = el % T::E32_CPR, rr0 = el / T::E32_CPR;
     const int col = n0 + wn * T::WTN + 4 * q;
+    const bool plane = SPLIT && OUT == kOutF32Partial; // a workspace plane
+    const int ld = plane ? pe.ws_ld : pe.ldc;
+    const void *base =
+        plane ? static_cast<const void *>(pe.ws + (size_t)part * (size_t)pe.M * (size_t)ld)
+              : pe.C;
     const __amdgpu_buffer_rsrc_t rc =
-        make_rsrc(rows_at(pe.C, m0, pe.ldc, 4), rows_bytes(m0, pe.M, pe.ldc, 4));
+        make_rsrc(rows_at(base, m0, ld, 4), rows_bytes(m0, pe.M, ld, 4));
     auto c_off = [&](int i, int s) -> uint32_t {
       const int trow = wm * T::WTM + 16 * i + s * T::E32_RPI + rr0;
       return m0 + trow < pe.M && col < pe.N
-                 ? ((uint32_t)trow * (uint32_t)pe.ldc + (uint32_t)col) * 4u
+                 ? ((uint32_t)trow * (uint32_t)ld + (uint32_t)col) * 4u
                  : kOob;
     };
     f32x4 old[OUT == kOutF32Accum ? PF : 1][NLD];
@@ -576,6 +599,27 @@ __device__ __forceinline__ void mfma16g_tile(const GemmParams &p, int m0, int n0
         *(TBK_LDS f32x4 *)(wl + r * T::E32_ROWB + (((4 * j + gg) ^ xr) * 16)) = acc[i][j];
         if (j & 1)
           __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (OUT == kOutF32Atomic) {
+        // 64 consecutive dwords per atomic: whole cache lines (the general
+        // loop's atomic epilogue)
+#pragma unroll
+        for (int t = 0; t < 16 * T::WTN / 64; ++t) {
+          const int rr = (t * 64 + el) / T::WTN, c = (t * 64 + el) % T::WTN;
+          const float v = *(const TBK_LDS float *)(
+              wl + rr * T::E32_ROWB + (((c / 4) ^ ((rr / T::E32_RPW) % T::E32_XM)) * 16) +
+              (c % 4) * 4);
+          const int trow = wm * T::WTM + 16 * i + rr, acol = n0 + wn * T::WTN + c;
+          const uint32_t off = m0 + trow < pe.M && acol < pe.N
+                                   ? ((uint32_t)trow * (uint32_t)ld + (uint32_t)acol) * 4u
+                                   : kOob;
+          __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(v, rc, off, 0, 0);
+        }
+        // the next block's writes are to these addresses: the other lanes'
+        // reads above stay before them
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        return;
       }
 #pragma unroll
       for (int s = 0; s < NLD; ++s) {
@@ -619,6 +663,17 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_mfma16g(GemmParams p) {
       __syncthreads(); // every wave read its staged epilogue back
     mfma16g_tile<BM, BN, BK, WGM, WGN, STAGES, OUT, EPI>(p, tile_m * BM, tile_n * BN, lds);
   }
+}
+
+// The programs of a split-K launch on the 16x16x32 loop.
+template <int BM, int BN, int BK, int WGM, int WGN, int STAGES, int OUT>
+__global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_mfma16g_split(GemmParams p) {
+  using T = Mfma16GTile<BM, BN, BK, WGM, WGN, STAGES>;
+  __shared__ u32x4 lds[T::LDS_BYTES / 16];
+  int tile_m, tile_n, part;
+  map_program(p, blockIdx.x, tile_m, tile_n, part);
+  mfma16g_tile<BM, BN, BK, WGM, WGN, STAGES, OUT, false, true>(p, tile_m * BM, tile_n * BN,
+                                                               lds, part);
 }
 
 } // namespace tbk

@@ -52,8 +52,9 @@ void desc_waits(const tb_gemm_desc *d, int64_t out[3]) {
   out[2] = d->entry->lgkm_loop;
 }
 
-// Validate a flattened config and bind it to a compiled instance.
-int create_desc(const tb_gemm_config &c, tb_gemm_desc **out) {
+// Validate a flattened config and bind it to a compiled instance; `part`:
+// a rectangle of a plan's launch, which may bind builds no plan names.
+int create_desc(const tb_gemm_config &c, tb_gemm_desc **out, bool part) {
   if (!out)
     return fail("tb_desc_create: out is NULL");
   *out = nullptr;
@@ -97,7 +98,7 @@ int create_desc(const tb_gemm_config &c, tb_gemm_desc **out) {
     return fail("group_m must be >= 1");
   if (c.mfma != TB_MFMA_32X32X16 && c.mfma != TB_MFMA_16X16X32)
     return fail("mfma must be TB_MFMA_32X32X16 or TB_MFMA_16X16X32");
-  if (c.mfma == TB_MFMA_16X16X32 && c.mapping == TB_MAP_SPLIT_K)
+  if (c.mfma == TB_MFMA_16X16X32 && c.mapping == TB_MAP_SPLIT_K && !part)
     return fail("the 16x16x32 instance has no split-K");
   const int64_t tiles_m = ceil_div(c.m, c.block_m);
   const int64_t tiles_n = ceil_div(c.n, c.block_n);
@@ -168,10 +169,11 @@ int create_desc(const tb_gemm_config &c, tb_gemm_desc **out) {
   tbk::KernelKey key{(int)c.block_m, (int)c.block_n, (int)c.block_k,
                      (int)c.wave_grid_m, (int)c.wave_grid_n, out_mode,
                      (int)c.stages, epi, (int)c.mfma};
-  const tbk::KernelEntry *e = tbk::find_kernel(key);
+  const bool split16 = c.mfma == TB_MFMA_16X16X32 && c.mapping == TB_MAP_SPLIT_K;
+  const tbk::KernelEntry *e = split16 ? tbk::find_split_kernel(key) : tbk::find_kernel(key);
   // an instance that spills to scratch is refused, as the plan refuses it
   // (the build-time table of the compiler's register report)
-  if (e) {
+  if (e && !split16) {
     tb::InstanceKey ik;
     ik.bm = c.block_m;
     ik.bn = c.block_n;
@@ -218,7 +220,7 @@ void choose_parts(tb_gemm_desc *d) {
   std::vector<tb_gemm_part> parts;
   for (const GridPart &g : split_grid(d->cfg)) {
     tb_gemm_desc *sub = nullptr;
-    if (create_desc(g.cfg, &sub)) {
+    if (create_desc(g.cfg, &sub, true)) {
       parts.clear();
       break;
     }
@@ -406,7 +408,7 @@ int tb_abi_version(void) { return TB_GFX950_ABI_VERSION; }
 int tb_desc_create(const tb_gemm_config *cfg, tb_gemm_desc **out) {
   if (!cfg)
     return fail("tb_desc_create: cfg is NULL");
-  return tbrt::create_desc(*cfg, out);
+  return tbrt::create_desc(*cfg, out, false);
 }
 
 int tb_desc_get_config(const tb_gemm_desc *desc, tb_gemm_config *out) {

@@ -34,8 +34,9 @@ struct tb_gemm_desc {
 };
 
 namespace tbrt {
-// Validates a flattened config and binds it to a compiled kernel instance.
-int create_desc(const tb_gemm_config &c, tb_gemm_desc **out);
+// Validates a flattened config and binds it to a compiled kernel instance
+// (`part`: one of a plan's launches, choose_parts).
+int create_desc(const tb_gemm_config &c, tb_gemm_desc **out, bool part);
 // Gives a planned descriptor the launches its problem runs best as
 // (grid_split.h); a descriptor made from a configuration runs that
 // configuration's own kernel.

@@ -147,11 +147,21 @@ std::vector<GridPart> split_grid(const tb_gemm_config &c) {
     // The splits stay the plan's. Of workgroups alone on their CUs, 2 stages
     // wait for loads that 3 have in flight (1024^2 x 8200 in 4 atomic splits
     // of 128x128: 36.1 -> 34.5 us, with a workspace 32.0 -> 29.6; 300 x 520 x
-    // 10000 in 12: 18.4 -> 16.8); short splits end before it matters.
+    // 10000 in 12: 18.4 -> 16.8); short splits end before it matters. 128x128
+    // tiles on 64-deep k-tiles run the 16x16x32 loop's build (34.1 -> 29.8
+    // us for the first of these).
     const int64_t k_tiles = ceil_div(c.k, c.block_k) / c.split_k;
-    if (c.stages != 2 || c.num_programs > kCus || k_tiles < 8)
+    if (c.num_programs > kCus || k_tiles < 8)
       return {};
     GridPart p{c};
+    if (c.block_m == 128 && c.block_n == 128 && c.block_k == 64 && c.wave_grid_m == 2 &&
+        c.wave_grid_n == 2) {
+      p.cfg.mfma = TB_MFMA_16X16X32;
+      p.cfg.stages = 3;
+      return {p};
+    }
+    if (c.stages != 2)
+      return {};
     p.cfg.stages = 3;
     return {p};
   }

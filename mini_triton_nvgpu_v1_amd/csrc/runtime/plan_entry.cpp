@@ -75,7 +75,7 @@ Planned configFromModule(tb::Module &m, const std::string &gpuArch) {
 // Bind the descriptor, then refuse it if the compiled kernel's waits are
 // not the ones the plan states.
 int bindPlanned(const Planned &p, tb_gemm_desc **out, const char *who) {
-  if (int rc = tbrt::create_desc(p.config, out))
+  if (int rc = tbrt::create_desc(p.config, out, false))
     return rc;
   if (p.waits.empty()) {
     tbrt::choose_parts(*out);

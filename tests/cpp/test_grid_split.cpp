@@ -46,7 +46,8 @@ int main() {
       CHECK(parts.empty());
     if (c.mapping == TB_MAP_SPLIT_K) { // as planned but for the stages
       for (const tbrt::GridPart &p : parts) {
-        CHECK(p.row0 == 0 && p.col0 == 0 && c.stages == 2 && p.cfg.stages == 3);
+        CHECK(p.row0 == 0 && p.col0 == 0 && p.cfg.stages == 3);
+        CHECK(c.stages == 2 || p.cfg.mfma == TB_MFMA_16X16X32);
         CHECK(p.cfg.m == c.m && p.cfg.n == c.n && p.cfg.split_k == c.split_k &&
               p.cfg.reduction == c.reduction && p.cfg.num_programs == c.num_programs);
       }

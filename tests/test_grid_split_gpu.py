@@ -13,6 +13,7 @@ from mini_triton_nvgpu_v1_amd import configs
 
 pytestmark = pytest.mark.gpu
 
+ATOMIC = {"tb.reduction-mode": '"split_k_parallel"'}
 BIG, MID, SMALL = (256, 256, 64), (128, 128, 64), (64, 64, 64)
 # (M, N, K, block, stages, options)
 CASES = [
@@ -26,7 +27,14 @@ CASES = [
     (4200, 4200, 328, BIG, 2, {"persistent": True, "num_ctas": 256}),
     (4200, 4200, 328, BIG, 2, {"c_f32": True}),
     (700, 1504, 2048, BIG, 2, {"c_f32": True}),
-    (300, 520, 5000, MID, 2, {"split_k": 4, "bias": "f16"}),  # 3 stages for 2
+    # split-K: 3 stages for 2, and 128x128 tiles on the 16x16x32 loop (splits of
+    # unequal length, a partial last k-tile, fewer rows than a wave tile)
+    (300, 520, 5000, (128, 64, 64), 2, {"split_k": 4, "bias": "f16"}),
+    (300, 520, 5000, MID, 2, {"split_k": 4, "bias": "f16", "activation": "relu"}),
+    (129, 136, 9224, MID, 3, {"split_k": 16}),
+    (7, 1032, 4096, MID, 2, {"split_k": 7, "c_f32": True}),
+    (1000, 776, 4168, MID, 2, {"split_k": 4, "c_f32": True, "module_attrs": ATOMIC}),
+    (129, 8, 9000, MID, 4, {"split_k": 3, "c_f32": True, "module_attrs": ATOMIC}),
 ]
 
 
@@ -56,9 +64,11 @@ def test_matches_planned_kernel(M, N, K, block, stages, options, device):
         desc.launch(a, b, c, ws, bias=bias)
         assert (buf[:256] == 3).all() and (buf[256 + M * N:] == 3).all()
         got.append(c)
+    if w.split_k > 1 and w.c_f32 and not w.module_attrs:
+        assert torch.equal(got[0], got[1])  # fixed reduction order, C added first
     if w.c_f32:
-        # the prior C is added before or after the products: one rounding of
-        # each running sum apart
+        # the prior C is added before or after the products (atomic splits in
+        # any order): one rounding of each running sum apart
         mag = a.float().abs() @ b.float().abs() + 3
         assert ((got[0] - got[1]).abs() <= (K + 2) * 2.0 ** -23 * mag).all()
         ref = a.double() @ b.double() + 3
