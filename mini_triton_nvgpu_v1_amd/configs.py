@@ -241,7 +241,7 @@ FUSED = [dataclasses.replace(ROOFLINE, name="gemm_4096_bias_gelu", bias="f16",
 F32_ACCUMULATE = [dataclasses.replace(ROOFLINE, name="gemm_4096_f32_accumulate",
                                       c_f32=True)]
 # Profiling rows (not bench lines): the 16x16x32 loop's 4-wave 128x128 tile at
-# 2048^3 (1024 tiles, four per CU), against the hand-scheduled 256x256 tile's
+# 2048^3 (256 tiles, one per CU), against the hand-scheduled 256x256 tile's
 # MFMA-busy fraction at 4096^3.
 PROFILE_ROWS = [Workload("gemm_2048_tile128", 2048, 2048, 2048, 0x5EED0007, NORMAL,
                          (128, 128, 64), num_waves=4, stages=3, group_m=8)]
