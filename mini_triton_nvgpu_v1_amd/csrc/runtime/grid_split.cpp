@@ -20,12 +20,12 @@
 //   256x256  7.3   0.955  1.37   68.1 / 68.6 / 95.1 us
 //   256x128  4.6   0.53   0.79   38.3 / 38.8 / 56.0
 //   128x128  4.1   0.333  0.455  25.4 / 25.8 / 33.1
-//    64x128  4.1   0.32   0.37   24.1 / 24.4 / 27.9
-//    64x64   3.6   0.27   0.275  20.6 / 20.8 / 21.2
+//    64x128  3.7   0.305  0.355  23.2 / 23.5 / 26.6
+//    64x64   3.25  0.255  0.262  19.6 / 19.7 / 20.1
 // The 64-row tiles fit a CU two or three times, so their further rounds
-// overlap: each costs 2.6 and 1.15 us and the K part 0.32 and 0.21 us per 64
-// of K and round (512 tiles of 64x128 at K = 1024 / 4096: 16.7 / 47.5 us,
-// 1024 of 64x64 at K = 64 / 1024 / 4096: 7.9 / 19.6 / 58.9).
+// overlap: each costs 2.2 and 0.92 us and the K part 0.3 and 0.195 us per 64
+// of K and round (1024 tiles, K = 64 / 1024 / 4096: 12.0 / 27.0 / 88.2 us on
+// 64x128, 7.0 / 17.6 / 55.3 on 64x64).
 // A choice has to be predicted 10% faster than the plan as it stands: the
 // constants reproduce the measured times to about 8%.
 #include "grid_split.h"
@@ -50,8 +50,8 @@ const Build kBuilds[] = {
     {256, 256, 2, 2, 2, TB_MFMA_16X16X32, 7.3, 0.955, 1.37, 0, 0},
     {256, 128, 4, 2, 3, TB_MFMA_16X16X32, 4.6, 0.53, 0.79, 0, 0},
     {128, 128, 2, 2, 3, TB_MFMA_16X16X32, 4.1, 0.333, 0.455, 0, 0},
-    {64, 128, 2, 4, 3, TB_MFMA_32X32X16, 4.1, 0.32, 0.37, 2.6, 0.32},
-    {64, 64, 2, 2, 3, TB_MFMA_32X32X16, 3.6, 0.27, 0.275, 1.15, 0.21},
+    {64, 128, 2, 4, 3, TB_MFMA_32X32X16, 3.7, 0.305, 0.355, 2.2, 0.3},
+    {64, 64, 2, 2, 3, TB_MFMA_32X32X16, 3.25, 0.255, 0.262, 0.92, 0.195},
 };
 
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -105,8 +105,8 @@ double over_build(const tb_gemm_config &c, const Build &b) {
 
 // The finest build within 5% of the fastest: what the constants leave out
 // (fused steps, an f32 C) is per element and spreads over more CUs
-// (1000 x 1496 x 712: 8.1 us predicted on 128x128, 8.2 on 64x128; 9.9 and
-// 8.5 measured).
+// (1000 x 1496 x 712: 8.1 us predicted on 128x128, 7.7 on 64x128; 9.9 and
+// 8.3 measured).
 const Build &fastest(int64_t m, int64_t n, int64_t k) {
   double least = grid_us(kBuilds[0], m, n, k);
   for (const Build &b : kBuilds)
