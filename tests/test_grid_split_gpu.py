@@ -75,3 +75,27 @@ def test_matches_planned_kernel(M, N, K, block, stages, options, device):
         assert ((got[0] - ref).abs() <= (K + 2) * 2.0 ** -24 * mag).all()
     else:
         assert torch.equal(got[0], got[1])
+
+
+def test_two_rectangles_in_a_graph(device):
+    """A captured launch of two rectangles, replayed with eager work between
+    the replays, gives the eager result each time."""
+    M, N, K = 4104, 4096, 136
+    print(f"grid split graph {M}x{N}x{K}", flush=True)
+    w = configs.Workload("w", M, N, K, 0, configs.NORMAL, BIG, num_waves=4, exact_tile=False)
+    desc = tb.plan_from_mlir(w.mlir())
+    a = torch.randn(M, K, device=device).half()
+    b = (torch.randn(K, N, device=device) / K ** 0.5).half()
+    c = torch.empty(M, N, device=device, dtype=torch.float16)
+    desc.launch(a, b, c)
+    eager = c.clone()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        desc.launch(a, b, c, stream=stream)
+    for _ in range(3):
+        c.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, eager)
