@@ -228,16 +228,20 @@ hipError_t launch_fill(void *dst, int64_t rows, int64_t cols, int64_t ld,
 
 // ---- instance registry ----------------------------------------------------
 // One table per shape and flavour (gemm_inst.hip), the hand-scheduled
-// 16x16x32 tables (f16 C; f32 C) and one 16x16x32 table per shape and
-// flavour of TBK_M16_SHAPES (gemm_inst_mfma16g.hip).
+// 16x16x32 tables (f16 C; f32 C) and one 16x16x32 table per shape, output
+// mode and flavour of TBK_M16_SHAPES (gemm_inst_mfma16g.hip).
 #define TBK_DECLARE(SHAPE)                                                      \
   const KernelEntry *entries_##SHAPE(int *n);                                  \
   const KernelEntry *entries_##SHAPE##_epi(int *n);
 TBK_SHAPES(TBK_DECLARE)
 #undef TBK_DECLARE
 #define TBK_DECLARE_M16(SHAPE)                                                  \
-  const KernelEntry *entries_m16_##SHAPE(int *n);                              \
-  const KernelEntry *entries_m16_##SHAPE##_epi(int *n);
+  const KernelEntry *entries_m16_##SHAPE##_o0(int *n);                         \
+  const KernelEntry *entries_m16_##SHAPE##_o1(int *n);                         \
+  const KernelEntry *entries_m16_##SHAPE##_o2(int *n);                         \
+  const KernelEntry *entries_m16_##SHAPE##_o0_epi(int *n);                     \
+  const KernelEntry *entries_m16_##SHAPE##_o1_epi(int *n);                     \
+  const KernelEntry *entries_m16_##SHAPE##_o2_epi(int *n);
 TBK_M16_SHAPES(TBK_DECLARE_M16)
 #undef TBK_DECLARE_M16
 const KernelEntry *entries_mfma16(int *n);
@@ -262,7 +266,9 @@ static const KernelEntry *preferred(const KernelEntry *e) {
 }
 
 #define TBK_TABLES(SHAPE) entries_##SHAPE, entries_##SHAPE##_epi,
-#define TBK_M16_TABLES(SHAPE) entries_m16_##SHAPE, entries_m16_##SHAPE##_epi,
+#define TBK_M16_TABLES(SHAPE)                                                  \
+  entries_m16_##SHAPE##_o0, entries_m16_##SHAPE##_o1, entries_m16_##SHAPE##_o2,         \
+      entries_m16_##SHAPE##_o0_epi, entries_m16_##SHAPE##_o1_epi, entries_m16_##SHAPE##_o2_epi,
 static const KernelEntry *(*const kTables[])(int *) = {
     TBK_SHAPES(TBK_TABLES) entries_mfma16, entries_mfma16_f32,
     TBK_M16_SHAPES(TBK_M16_TABLES)};

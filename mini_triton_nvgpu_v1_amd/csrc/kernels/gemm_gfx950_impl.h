@@ -145,29 +145,33 @@ __device__ __forceinline__ void acc_read_fence(f32x4 (&acc)[TI][TJ]) {
 // pass through an asm (no instruction) that differs per (activation, clamp):
 // the variants then share no accumulator read that the compiler could hoist
 // above the dispatch, where it would hold the whole tile in VGPRs at once.
+// The block index is an int that is a constant once inlined, so a block's code
+// is one function per variant and not one per block and variant (the build
+// compiles it once, not 8 to 16 times).
 template <bool EPI, bool ONCE, int NB, int TJ, class F>
 __device__ __forceinline__ void epi_for_blocks(const GemmParams &pe, f32x4 (&acc)[NB][TJ],
                                                F &&block) {
-  auto variant = [&](auto i_c, auto act_c, auto clamp_c) {
+  auto variant = [&](int i, auto act_c, auto clamp_c) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < TJ; ++j)
       asm volatile("; fused epilogue variant %1 %2"
-                   : "+a"(acc[decltype(i_c)::value][j])
+                   : "+a"(acc[i][j])
                    : "i"(decltype(act_c)::value), "i"(decltype(clamp_c)::value ? 1 : 0));
     __builtin_amdgcn_sched_barrier(0); // nothing scheduled above it
-    block(i_c, act_c, clamp_c);
+    block(i, act_c, clamp_c);
   };
   if constexpr (EPI && ONCE)
     epi_dispatch(pe.epi_act, pe.epi_clamp, [&](auto act_c, auto clamp_c) {
-      static_for<NB>([&](auto i_c) { variant(i_c, act_c, clamp_c); });
+      static_for<NB>([&](auto i_c) { variant(decltype(i_c)::value, act_c, clamp_c); });
     });
   else
     static_for<NB>([&](auto i_c) {
+      constexpr int i = decltype(i_c)::value;
       if constexpr (EPI)
         epi_dispatch(pe.epi_act, pe.epi_clamp,
-                     [&](auto act_c, auto clamp_c) { variant(i_c, act_c, clamp_c); });
+                     [&](auto act_c, auto clamp_c) { variant(i, act_c, clamp_c); });
       else
-        block(i_c, std::integral_constant<int, 0>{}, std::integral_constant<bool, false>{});
+        block(i, std::integral_constant<int, 0>{}, std::integral_constant<bool, false>{});
     });
 }
 
@@ -519,21 +523,17 @@ __device__ __forceinline__ void mfma16_tile(const GemmParams &p, int m0, int n0,
   const uint32_t a_bytes = rows_bytes(m0, p.M, p.lda, 2);
   const uint32_t b_bytes = (uint32_t)p.K * (uint32_t)p.ldb * 2u;
   const uint32_t wlds = lds0 + wave * 1024u;
-  // load l of k-tile kt into ring slot ST (l is a constant once unrolled:
-  // the LDS offset becomes the literal of the M0 add)
-  auto load = [&](const u32x4 &ra, const u32x4 &rb, int kt, auto st_c, int l) {
+  // load L of k-tile kt into ring slot ST (constants: the LDS offset is the
+  // literal of the M0 add)
+  auto load = [&](const u32x4 &ra, const u32x4 &rb, int kt, auto st_c, auto l_c) {
     constexpr uint32_t base = decltype(st_c)::value * SLOT;
-    static_for<16>([&](auto l_c) {
-      constexpr int L = decltype(l_c)::value;
-      if (L == l) {
-        if constexpr (L < 8)
-          load_lds16_at<base + L * 4096u>(ra, wlds, L * 32 < a_rows_left ? a_voff : kOob,
-                                          (uint32_t)kt * a_ktile + L * a_round);
-        else
-          load_lds16_at<base + B_AT + (L - 8) * 4096u>(
-              rb, wlds, (L & 1) ? b_voff1 : b_voff0, (uint32_t)kt * b_ktile + (L - 8) * b_round);
-      }
-    });
+    constexpr int L = decltype(l_c)::value;
+    if constexpr (L < 8)
+      load_lds16_at<base + L * 4096u>(ra, wlds, L * 32 < a_rows_left ? a_voff : kOob,
+                                      (uint32_t)kt * a_ktile + L * a_round);
+    else
+      load_lds16_at<base + B_AT + (L - 8) * 4096u>(
+          rb, wlds, (L & 1) ? b_voff1 : b_voff0, (uint32_t)kt * b_ktile + (L - 8) * b_round);
   };
   using S0 = std::integral_constant<int, 0>;
   using S1 = std::integral_constant<int, 1>;
@@ -604,12 +604,10 @@ __device__ __forceinline__ void mfma16_tile(const GemmParams &p, int m0, int n0,
     static_for<64>([&](auto m_c) {
       constexpr int m = decltype(m_c)::value;
       mfma(0, m, first);
-      static_for<24>([&](auto o_c) {
-        constexpr int o = decltype(o_c)::value;
-        if constexpr (Sched::slot_ks0(o) == m)
-          rd(1, st, 1, o);
-      });
-      extra(m);
+      constexpr int o = Sched::op_ks0(m);
+      if constexpr (o >= 0)
+        rd(1, st, 1, o);
+      extra(m_c);
       __builtin_amdgcn_sched_barrier(0);
     });
   };
@@ -619,16 +617,16 @@ __device__ __forceinline__ void mfma16_tile(const GemmParams &p, int m0, int n0,
       constexpr int m = decltype(m_c)::value;
       if constexpr (m >= decltype(lo_c)::value && m < decltype(hi_c)::value) {
         mfma(1, m, false);
-        extra(m);
+        extra(m_c);
         __builtin_amdgcn_sched_barrier(0);
       }
     });
   };
-  auto kstep1 = [&](auto lo_c, auto hi_c) { kstep1x(lo_c, hi_c, [](int) {}); };
+  auto kstep1 = [&](auto lo_c, auto hi_c) { kstep1x(lo_c, hi_c, [](auto) {}); };
   using Z = std::integral_constant<int, 0>;
   using Q = std::integral_constant<int, BQ>;
   using E = std::integral_constant<int, 64>;
-  auto nothing = [](int) {};
+  auto nothing = [](auto) {};
 
   // f32 C += A*B: the prior C is added into the accumulators during the
   // first 16 loop bodies instead of after the loop, so its 64 MB (at 4096^3)
@@ -663,18 +661,15 @@ __device__ __forceinline__ void mfma16_tile(const GemmParams &p, int m0, int n0,
   };
   // the add of body q at slot s of its first k step (s < 64) or of the next
   // (s - 64): tile s - 8
-  auto c_add = [&](auto q_c, int s) {
-    constexpr int q = decltype(q_c)::value;
-    static_for<4>([&](auto t_c) {
-      constexpr int t = decltype(t_c)::value, mm = 4 * q + t;
-      if (s == mm + 8) {
-        acc[mm >> 3][mm & 7] += cbuf[q & 1][t];
-        // the sum back in its AGPRs in this slot: left to the compiler, the
-        // v_accvgpr_write sinks to right before the tile's next asm MFMA,
-        // which then reads srcC without the VALU-write wait states
-        asm volatile("" : "+a"(acc[mm >> 3][mm & 7]));
-      }
-    });
+  auto c_add = [&](auto q_c, auto s_c) {
+    constexpr int q = decltype(q_c)::value, mm = decltype(s_c)::value - 8, t = mm - 4 * q;
+    if constexpr (t >= 0 && t < 4) {
+      acc[mm >> 3][mm & 7] += cbuf[q & 1][t];
+      // the sum back in its AGPRs in this slot: left to the compiler, the
+      // v_accvgpr_write sinks to right before the tile's next asm MFMA,
+      // which then reads srcC without the VALU-write wait states
+      asm volatile("" : "+a"(acc[mm >> 3][mm & 7]));
+    }
   };
   if constexpr (C_IN_LOOP) {
     if (c_in_loop)
@@ -686,12 +681,8 @@ __device__ __forceinline__ void mfma16_tile(const GemmParams &p, int m0, int n0,
     const u32x4 ra = rsrc_dwords(a_tile, a_bytes), rb = rsrc_dwords(p.B, b_bytes);
     const u32x4 ra1 = rsrc_dwords(a_tile, nk > 1 ? a_bytes : 0u);
     const u32x4 rb1 = rsrc_dwords(p.B, nk > 1 ? b_bytes : 0u);
-#pragma unroll
-    for (int l = 0; l < 16; ++l)
-      load(ra, rb, 0, S0{}, l);
-#pragma unroll
-    for (int l = 0; l < 16; ++l)
-      load(ra1, rb1, 1, S1{}, l);
+    static_for<16>([&](auto l_c) { load(ra, rb, 0, S0{}, l_c); });
+    static_for<16>([&](auto l_c) { load(ra1, rb1, 1, S1{}, l_c); });
   }
   wait_vmcnt<kMfma16VmPrologue>();
   barrier();
@@ -718,28 +709,27 @@ __device__ __forceinline__ void mfma16_tile(const GemmParams &p, int m0, int n0,
     static_for<64 - BQ>([&](auto s_c) {
       constexpr int m = BQ + decltype(s_c)::value;
       mfma(1, m, false);
-      static_for<Sched::NREAD>([&](auto o_c) {
-        constexpr int o = decltype(o_c)::value;
-        if constexpr (Sched::slot_ks1(o) == m)
-          rd(0, Sn, 0, o);
-      });
+      constexpr int o = Sched::op_ks1(m);
+      if constexpr (o >= 0)
+        rd(0, Sn, 0, o);
       if constexpr (((m - BQ) % LS) == 0)
-        load(ra, rb, it + 2, stage, (m - BQ) / LS);
+        load(ra, rb, it + 2, stage, std::integral_constant<int, (m - BQ) / LS>{});
       __builtin_amdgcn_sched_barrier(0);
     });
     constexpr int NB = (64 - BQ + LS - 1) / LS; // refill loads issued before k-tile it+1
     constexpr int OFF = NB * LS - (64 - BQ);    // slot of k-tile it+1 with its first load
     static_assert(OFF + (16 - NB - 1) * LS < 64, "refill fits one k-tile");
-    auto refill = [&](int m) {
-      if (m >= OFF && ((m - OFF) % LS) == 0 && NB + (m - OFF) / LS < 16)
-        load(ra, rb, it + 2, stage, NB + (m - OFF) / LS);
-      k0(m);
+    auto refill = [&](auto m_c) {
+      constexpr int m = decltype(m_c)::value;
+      if constexpr (m >= OFF && ((m - OFF) % LS) == 0 && NB + (m - OFF) / LS < 16)
+        load(ra, rb, it + 2, stage, std::integral_constant<int, NB + (m - OFF) / LS>{});
+      k0(m_c);
     };
     kstep0(Sn, refill, false);
     kstep1x(Z{}, Q{}, k1);
   };
   auto body = [&](int it, auto stage) {
-    auto none = [](int) {};
+    auto none = [](auto) {};
     body_h(it, stage, []() {}, none, none);
   };
   int it = 0;
@@ -753,7 +743,10 @@ __device__ __forceinline__ void mfma16_tile(const GemmParams &p, int m0, int n0,
               if constexpr (q + 1 < 16)
                 c_load(std::integral_constant<int, q + 1>{});
             },
-            [&](int m) { c_add(q_c, m); }, [&](int m) { c_add(q_c, m + 64); });
+            [&](auto m_c) { c_add(q_c, m_c); },
+            [&](auto m_c) {
+              c_add(q_c, std::integral_constant<int, decltype(m_c)::value + 64>{});
+            });
       });
       it = 16;
     }
@@ -808,20 +801,15 @@ __device__ __forceinline__ void mfma16_tile(const GemmParams &p, int m0, int n0,
     // while block i+1's conversions (and fused steps) execute. The region is
     // this wave's alone and a wave's LDS operations complete in order, so no
     // barrier separates a block's writes from its reads.
-    auto block = [&](auto i_c, auto act_c, auto clamp_c) {
-      constexpr int i = decltype(i_c)::value;
+    auto block = [&](int i, auto act_c, auto clamp_c) __attribute__((always_inline)) {
       constexpr int ACT = decltype(act_c)::value;
       constexpr bool CLAMP = decltype(clamp_c)::value;
       const int r = 16 * i + (el & 15);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        float x[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          x[e] = acc[i][j][e];
-          if constexpr (EPI)
-            x[e] = epi_apply_t<ACT, CLAMP>(x[e], bv[j][e], lo, hi);
-        }
+        f32x4 x = acc[i][j];
+        if constexpr (EPI)
+          x = epi_apply4_t<ACT, CLAMP>(x, bv[j], lo, hi);
         u32x2 v;
         v[0] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)x[0]) |
                ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)x[1]) << 16);
@@ -893,8 +881,7 @@ __device__ __forceinline__ void mfma16_tile(const GemmParams &p, int m0, int n0,
     TBK_LDS char *wl = (TBK_LDS char *)(TBK_LDS void *)lds + wave * 32768;
     const float lo = (pe.epi_clamp & 1) ? pe.clamp_lo : -__builtin_inff();
     const float hi = (pe.epi_clamp & 2) ? pe.clamp_hi : __builtin_inff();
-    auto block = [&](auto i_c, auto act_c, auto clamp_c) {
-      constexpr int i = decltype(i_c)::value;
+    auto block = [&](int i, auto act_c, auto clamp_c) __attribute__((always_inline)) {
       constexpr int ACT = decltype(act_c)::value;
       constexpr bool CLAMP = decltype(clamp_c)::value;
       TBK_LDS char *blk = wl + (i & 3) * 8192;
@@ -914,9 +901,7 @@ __device__ __forceinline__ void mfma16_tile(const GemmParams &p, int m0, int n0,
             v += old[i % PF][t];
         }
         if constexpr (EPI) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            v[e] = epi_apply_t<ACT, CLAMP>(v[e], bias[e], lo, hi);
+          v = epi_apply4_t<ACT, CLAMP>(v, bias, lo, hi);
         }
         // a plain f32 C is written once and not read again by this kernel
         // (non-temporal); C += A*B keeps the default policy

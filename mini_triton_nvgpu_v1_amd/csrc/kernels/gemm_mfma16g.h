@@ -117,9 +117,9 @@ struct Mfma16GTile {
   static constexpr int SPREAD = STAGES == 2 ? NSLOT * 5 / 8 : NSLOT - NSLOT / 8;
   static constexpr int load_slot(int l) { return l * SPREAD / LPT; }
   // the k-th read op (or load) placed in slot m, -1 if none: per-slot
-  // tables, so the unrolled slots instantiate only what they issue
-  static constexpr int RPS = NR / NM + 2; // bound on read ops per slot
-  static constexpr int LPS = LPT / SPREAD + 2; // bound on loads per body slot
+  // tables, so the unrolled slots instantiate only what they issue (a lambda
+  // per slot and candidate op took most of the build's time)
+  static constexpr int PER_SLOT = 2; // bound on read ops, and on loads, per slot
   static constexpr int mid_op(int m, int k) {
     for (int o = 0, c = 0; o < NR; ++o)
       if (slot_mid(o) == m && c++ == k)
@@ -193,10 +193,10 @@ struct Mfma16GTile {
   static_assert(SPREAD >= 1 && SPREAD <= NSLOT, "refill within one body");
   static constexpr bool tables_cover() {
     for (int m = 0; m < NM; ++m)
-      if (mid_op(m, RPS - 1) >= 0 || last_op(m, RPS - 1) >= 0)
+      if (mid_op(m, PER_SLOT) >= 0 || last_op(m, PER_SLOT) >= 0)
         return false;
     for (int s2 = 0; s2 < NSLOT; ++s2)
-      if (load_at(s2, LPS - 1) >= 0)
+      if (load_at(s2, PER_SLOT) >= 0)
         return false;
     return true;
   }
@@ -362,13 +362,15 @@ __device__ __forceinline__ void mfma16g_tile(const GemmParams &p, int m0, int n0
       constexpr int M = decltype(m_c)::value;
       if constexpr (M >= decltype(lo_c)::value && M < decltype(hi_c)::value) {
         mfma(BUF::value, M, decltype(first_c)::value);
-        if constexpr (KSI + 1 < KS)
-          static_for<T::RPS>([&](auto k_c) {
-            constexpr int O = T::mid_op(M, decltype(k_c)::value);
-            if constexpr (O >= 0)
-              rd(std::integral_constant<int, 1>{}, std::integral_constant<int, ST>{},
-                 std::integral_constant<int, KSI + 1>{}, std::integral_constant<int, O>{});
-          });
+        if constexpr (KSI + 1 < KS) {
+          constexpr int O0 = T::mid_op(M, 0), O1 = T::mid_op(M, 1);
+          using B1 = std::integral_constant<int, 1>;
+          using KN = std::integral_constant<int, KSI + 1>;
+          if constexpr (O0 >= 0)
+            rd(B1{}, std::integral_constant<int, ST>{}, KN{}, std::integral_constant<int, O0>{});
+          if constexpr (O1 >= 0)
+            rd(B1{}, std::integral_constant<int, ST>{}, KN{}, std::integral_constant<int, O1>{});
+        }
         extra(m_c);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -394,21 +396,22 @@ __device__ __forceinline__ void mfma16g_tile(const GemmParams &p, int m0, int n0
     // body slot s: s = m - BQ in the last k step of k-tile it, then
     // NM - BQ + ks NM + m in k-tile it+1
     auto refill_at = [&](auto s_c) {
-      static_for<T::LPS>([&](auto k_c) {
-        constexpr int L = T::load_at(decltype(s_c)::value, decltype(k_c)::value);
-        if constexpr (L >= 0)
-          load(ra, rb, it + STAGES, std::integral_constant<int, SC>{},
-               std::integral_constant<int, L>{});
-      });
+      constexpr int S = decltype(s_c)::value, L0 = T::load_at(S, 0), L1 = T::load_at(S, 1);
+      using SLOT = std::integral_constant<int, SC>;
+      if constexpr (L0 >= 0)
+        load(ra, rb, it + STAGES, SLOT{}, std::integral_constant<int, L0>{});
+      if constexpr (L1 >= 0)
+        load(ra, rb, it + STAGES, SLOT{}, std::integral_constant<int, L1>{});
     };
     using BN0 = decltype(buf_of(QN{}, Z{}));
     kstep(q_c, LAST{}, QB{}, ENDS{}, first_c, [&](auto m_c) {
       constexpr int M = decltype(m_c)::value;
-      static_for<T::RPS>([&](auto k_c) {
-        constexpr int O = T::last_op(M, decltype(k_c)::value);
-        if constexpr (O >= 0)
-          rd(BN0{}, std::integral_constant<int, SN>{}, Z{}, std::integral_constant<int, O>{});
-      });
+      constexpr int O0 = T::last_op(M, 0), O1 = T::last_op(M, 1);
+      using SNEXT = std::integral_constant<int, SN>;
+      if constexpr (O0 >= 0)
+        rd(BN0{}, SNEXT{}, Z{}, std::integral_constant<int, O0>{});
+      if constexpr (O1 >= 0)
+        rd(BN0{}, SNEXT{}, Z{}, std::integral_constant<int, O1>{});
       refill_at(std::integral_constant<int, M - BQ>{});
     });
     static_for<KS>([&](auto ks_c) {
@@ -509,19 +512,14 @@ __device__ __forceinline__ void mfma16g_tile(const GemmParams &p, int m0, int n0
     const int xr = (r / T::E16_RPW) % T::E16_XM, hs = (r >> 3) & 1;
     const int q = el % T::E16_CPR, rr0 = el / T::E16_CPR;
     const int col = n0 + wn * T::WTN + 8 * q;
-    auto block = [&](auto i_c, auto act_c, auto clamp_c) {
-      constexpr int i = decltype(i_c)::value;
+    auto block = [&](int i, auto act_c, auto clamp_c) __attribute__((always_inline)) {
       constexpr int ACT = decltype(act_c)::value;
       constexpr bool CLAMP = decltype(clamp_c)::value;
 #pragma unroll
       for (int j = 0; j < TJ; ++j) {
-        float x[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          x[e] = acc[i][j][e];
-          if constexpr (EPI)
-            x[e] = epi_apply_t<ACT, CLAMP>(x[e], bv[j][e], lo, hi);
-        }
+        f32x4 x = acc[i][j];
+        if constexpr (EPI)
+          x = epi_apply4_t<ACT, CLAMP>(x, bv[j], lo, hi);
         u32x2 v;
         v[0] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)x[0]) |
                ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)x[1]) << 16);
@@ -590,8 +588,7 @@ __device__ __forceinline__ void mfma16g_tile(const GemmParams &p, int m0, int n0
     barrier(); // every wave is past its last fragment read and load
     const int r = el & 15, gg = el >> 4;
     const int xr = (r / T::E32_RPW) % T::E32_XM;
-    auto block = [&](auto i_c, auto act_c, auto clamp_c) {
-      constexpr int i = decltype(i_c)::value;
+    auto block = [&](int i, auto act_c, auto clamp_c) __attribute__((always_inline)) {
       constexpr int ACT = decltype(act_c)::value;
       constexpr bool CLAMP = decltype(clamp_c)::value;
 #pragma unroll
@@ -629,9 +626,7 @@ __device__ __forceinline__ void mfma16g_tile(const GemmParams &p, int m0, int n0
         if constexpr (OUT == kOutF32Accum)
           v += old[i % PF][s];
         if constexpr (EPI) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            v[e] = epi_apply_t<ACT, CLAMP>(v[e], bias[e], lo, hi);
+          v = epi_apply4_t<ACT, CLAMP>(v, bias, lo, hi);
         }
         // a plain f32 C is written once (non-temporal); C += A*B keeps the
         // default policy

@@ -45,6 +45,26 @@ struct Mfma16Schedule {
   static constexpr int slot_ks0(int o) { return RNUM * o / RDEN; }
   static constexpr int slot_ks1(int o) { return BQ + R1NUM * o / R1DEN; }
 
+  // the read op of slot m, or -1 (a slot carries at most one)
+  static constexpr int op_ks0(int m) {
+    for (int o = 0; o < NREAD; ++o)
+      if (slot_ks0(o) == m)
+        return o;
+    return -1;
+  }
+  static constexpr int op_ks1(int m) {
+    for (int o = 0; o < NREAD; ++o)
+      if (slot_ks1(o) == m)
+        return o;
+    return -1;
+  }
+  static constexpr bool one_read_per_slot() {
+    for (int o = 0; o < NREAD; ++o)
+      if (op_ks0(slot_ks0(o)) != o || op_ks1(slot_ks1(o)) != o)
+        return false;
+    return true;
+  }
+
   static constexpr int last_read(bool a, int idx) {
     int last = -1;
     for (int m = 0; m < NSLOT; ++m)
@@ -97,6 +117,7 @@ struct Mfma16Schedule {
   static_assert(covers_every_tile_once(), "(a) first-MFMA srcC = 0 needs one MFMA per tile");
   static_assert(reads_fit(), "fragment reads must fall inside their k step (and after the "
                              "barrier for the next k-tile's reads)");
+  static_assert(one_read_per_slot(), "a slot carries at most one fragment read");
   static_assert(slot_ks1(NREAD - 1) < NSLOT, "the next k-tile's reads must fit after the barrier");
   static_assert(min_rewrite_distance() >= MIN_REWRITE_SLOTS,
                 "(c) a fragment register rewritten too soon after its last MFMA read");

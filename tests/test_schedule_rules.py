@@ -44,6 +44,8 @@ def test_kernel_schedule_builds(tmp_path):
     ("16, 1, 4, 24, 2, 1", "(c) a fragment register rewritten too soon"),
     # the next k-tile's reads would run past the k step
     ("24, 8, 3, 24, 2, 1", "the next k-tile's reads must fit after the barrier"),
+    # two of k step 1's reads in one slot: the kernel issues one per slot
+    ("8, 1, 2, 24, 7, 3", "a slot carries at most one fragment read"),
     # k step 1's reads spread past the end of k step 0
     ("16, 3, 1, 24, 2, 1", "fragment reads must fall inside their k step"),
 ])
