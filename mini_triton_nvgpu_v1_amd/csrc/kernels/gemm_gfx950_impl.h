@@ -926,6 +926,18 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_kernel(GemmParams p) {
   using T = GemmTile<BM, BN, BK, WGM, WGN, STAGES, SPREAD_REQ>;
   constexpr int NW = T::NW, KCH = T::KCH, BNC = T::BNC, TM = T::TM, TN = T::TN,
                 KSTEPS = T::KSTEPS, NMFMA = T::NMFMA, LA = T::LA, LPT = T::LPT;
+  // Burst schedule: the last STAGES k-tiles run a copy of the loop body of
+  // their own (below), which takes 5 to 25 more registers. Not where they cost
+  // a workgroup per CU that LDS has room for: 32-deep k-tiles on wave tiles
+  // of more than one MFMA, or with fused steps, and fused steps on 64-row
+  // wave tiles in 2 stages. Against no copy, with several workgroups per CU:
+  // 3000^2 x 1000 on 64x128x32 in 1x4 waves 38.9 -> 40.7 us, with GELU 42.2 ->
+  // 50.4; 64x128x64 with SiLU in 2 stages 39.7 -> 43.4, but in 3 stages, where
+  // LDS holds 2 workgroups anyway, 40.1 -> 39.7 (4096^2 x 128: 30.1 -> 25.5).
+  constexpr bool STEPS_FIRST = EPI && OUT != kOutF32Accum; // steps on the accumulators
+  constexpr bool TAIL_COPY =
+      NW < 4 || !((BK == 32 && (NMFMA >= 2 || (STEPS_FIRST && NW == 4))) ||
+                  (STEPS_FIRST && STAGES == 2 && TM >= 2));
   __shared__ u32x4 lds[STAGES * T::STAGE + T::SCRATCH_CHUNKS];
   auto stage_base = [&](int st) -> u32x4 * { return lds + st * T::STAGE; };
 
@@ -1188,18 +1200,18 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_kernel(GemmParams p) {
         if (T::load_off(l) < T::AFTER)
           issue_load(kt0 + STAGES - 1, STAGES - 1, l);
     } else {
-      // only the k-tiles there are: a short K would otherwise wait for loads
-      // of zeros
+      // with the copy only the k-tiles there are: a short K would otherwise
+      // wait for loads of zeros
 #pragma unroll
       for (int st = 0; st < STAGES; ++st)
-        if (st == 0 || st < nk)
+        if (!TAIL_COPY || st == 0 || st < nk)
           issue_tile(kt0 + st, st);
     }
     // burst schedule: the wait for a k-tile behind which `tiles` more are in
     // flight, and EXTRA other loads
     auto wait_tiles = [&](int tiles, auto extra_c) {
       constexpr int EXTRA = decltype(extra_c)::value;
-      if (tiles >= STAGES - 1)
+      if (!TAIL_COPY || tiles >= STAGES - 1)
         wait_vmcnt<(STAGES - 1) * LPT + EXTRA>();
       else if (STAGES > 2 && tiles == STAGES - 2)
         wait_vmcnt<(STAGES - 2) * LPT + EXTRA>();
@@ -1292,15 +1304,15 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_kernel(GemmParams p) {
         s = s_next;
       }
     } else {
-      // Burst schedule. The k-tiles whose refill exists run the loop; the
-      // last STAGES ones run a copy that waits for, reads and loads only
-      // what there is (K up to a few k-tiles, where lookahead loads of zeros
-      // and the barrier after the last k-tile were 0.3 us of a 3 us kernel:
-      // 448x288x64 on 64x64x64, f32 C += A*B: 3.22 -> 2.93 us; the tail's
-      // branches in the loop itself cost 7% at K = 4096). After a barrier
-      // the refill goes out before the fragment reads (1024^2 x 4096, 64x64x64
-      // in 3 stages: 21.3 -> 20.1; 64x128x64 on 1x4 waves: 26.8 -> 25.7; in 2
-      // stages 31.2 -> 31.1).
+      // Burst schedule. With TAIL_COPY the k-tiles whose refill exists run
+      // the loop, and the last STAGES ones a copy that waits for, reads and
+      // loads only what there is (1024^2 on 64x64x64, K = 64: 4.1 -> 3.9 us;
+      // 128x64x64 in 3 stages, K = 256: 5.5 -> 5.1; 64x64x64 at 4096^2 x 128:
+      // 20.8 -> 18.4; the tail's branches in the loop itself cost 7% at K =
+      // 4096); without it every k-tile runs the loop, whose lookahead loads
+      // past the last k-tile are zeros. After a barrier the refill goes out
+      // before the fragment reads (1024^2 x 4096, 64x64x64 in 3 stages: 21.3 ->
+      // 20.1; 64x128x64 on 1x4 waves: 26.8 -> 25.7; in 2 stages 31.2 -> 31.1).
       auto ktile = [&](int it, auto tail_c) {
         constexpr bool TAIL = decltype(tail_c)::value;
         const int s_next = s + 1 == STAGES ? 0 : s + 1;
@@ -1336,11 +1348,13 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_kernel(GemmParams p) {
         s = s_next;
       };
       int it = 0;
-      for (; it + STAGES < nk; ++it)
+      for (; it + (TAIL_COPY ? STAGES : 0) < nk; ++it)
         ktile(it, std::integral_constant<bool, false>{});
+      if constexpr (TAIL_COPY) {
 #pragma nounroll
-      for (; it < nk; ++it)
-        ktile(it, std::integral_constant<bool, true>{});
+        for (; it < nk; ++it)
+          ktile(it, std::integral_constant<bool, true>{});
+      }
     }
 
     // Drain the (out-of-range, zero) loads still in flight into LDS so none
