@@ -139,10 +139,16 @@ int tb_desc_create(const tb_gemm_config *cfg, tb_gemm_desc **out);
  *
  * A launch of a planned descriptor may run the problem on another compiled
  * tile, or as two rectangles of C, where the planned grid would leave compute
- * units idle (csrc/runtime/grid_split.h): every tile adds an element's
- * products in the same order, so C is the same. The descriptor's config and
- * kernel name stay the plan's; tb_desc_create with that config runs exactly
- * that kernel. */
+ * units idle (csrc/runtime/grid_split.h). Every tile adds an element's
+ * products in the same order, so an f16 C, a plain f32 C and a split-K with a
+ * workspace have the same bits. f32 C += A*B: the planned kernel of the
+ * 256x256x64 tile on 4 waves and 2 stages adds the prior C within its first
+ * k-tiles (K a multiple of 64, at least 1152), a small wave tile not staged
+ * through LDS first of all, the others last; a launch never adds it earlier
+ * than the planned kernel, and where it adds it later, sums differ by their
+ * rounding. Atomic split-K has no fixed order on any kernel. The descriptor's
+ * config and kernel name stay the plan's; tb_desc_create with that config
+ * runs exactly that kernel. */
 int tb_plan_from_mlir(const char *mlir, size_t len, const char *gpu_arch,
                       tb_gemm_desc **out);
 

@@ -433,7 +433,8 @@ class GemmDesc:
 def plan_from_mlir(text: str, gpu_arch: str = "gfx950") -> GemmDesc:
     """Run the tb plan pipeline on a module holding one tb.matmul. A launch of
     the descriptor may run the problem on another compiled tile, or as two
-    rectangles of C, where the planned grid would leave compute units idle;
+    rectangles of C, where the planned grid would leave compute units idle
+    (include/tb_gfx950.h says what that leaves the same);
     ``GemmDesc.from_config(desc.config)`` runs the planned kernel itself."""
     data = text.encode()
     h = ctypes.c_void_p()

@@ -6,8 +6,8 @@
 // kept 24 of 256 CUs busy for 30 us, and 320 of them (5000 x 4096 x 4104)
 // took two rounds, the second a quarter full, 178 us. C does not depend on
 // the tile: every build adds the products of an element in the same k order
-// in f32 (bit-identical for f16 and plain f32 results; f32 C += A*B may round
-// its one addition of the prior C elsewhere). So the launch of a plan may
+// in f32 (bit-identical for f16 and plain f32 results; for f32 C += A*B see
+// adds_c_early). So the launch of a plan may
 // run the same problem on another tile, or cut it in two rectangles: the rows
 // (or columns) that fill whole rounds on the planned tile, and the rest on a
 // tile that spreads it over the chip.
@@ -103,17 +103,35 @@ double over_build(const tb_gemm_config &c, const Build &b) {
   return tiles <= kCus && c.k >= 1024 && (c.stages == 2 || c.num_waves < 4) ? 1.2 : 1;
 }
 
+// f32 C += A*B: the 256x256 build adds the prior C inside its first 16
+// k-tiles (whole k-tiles only, at least 18 of them), the other builds after
+// the last one. Every sum after the addition rounds at the larger magnitude:
+// at K = 4096 the error against f64 is 1.6 times that of adding C last. So a
+// plan on another tile, whose kernel adds C last (or, on small wave tiles not
+// staged through LDS, first), never moves there.
+bool adds_c_early(const Build &b, const tb_gemm_config &c) {
+  return c.acc_init == TB_ACC_INIT_LOAD_C && b.bm == 256 && b.bn == 256 && c.k % 64 == 0 &&
+         c.k >= 18 * 64;
+}
+
 // The finest build within 5% of the fastest: what the constants leave out
 // (fused steps, an f32 C) is per element and spreads over more CUs
 // (1000 x 1496 x 712: 8.1 us predicted on 128x128, 7.7 on 64x128; 9.9 and
-// 8.3 measured).
-const Build &fastest(int64_t m, int64_t n, int64_t k) {
-  double least = grid_us(kBuilds[0], m, n, k);
+// 8.3 measured). `c`: the plan, whose K it is and whose C += A*B rounding the
+// build may not worsen.
+const Build &fastest(const tb_gemm_config &c, int64_t m, int64_t n) {
+  auto allowed = [&](const Build &b) {
+    return !adds_c_early(b, c) || (build_of(c) == &b && is_build(c, b));
+  };
+  const Build *best = nullptr;
+  double least = 0;
   for (const Build &b : kBuilds)
-    least = std::min(least, grid_us(b, m, n, k));
-  const Build *best = &kBuilds[0];
+    if (allowed(b) && (!best || grid_us(b, m, n, c.k) < least)) {
+      best = &b;
+      least = grid_us(b, m, n, c.k);
+    }
   for (const Build &b : kBuilds) // coarse to fine
-    if (grid_us(b, m, n, k) <= 1.05 * least)
+    if (allowed(b) && grid_us(b, m, n, c.k) <= 1.05 * least)
       best = &b;
   return *best;
 }
@@ -179,7 +197,7 @@ std::vector<GridPart> split_grid(const tb_gemm_config &c) {
   std::vector<GridPart> best;
 
   // the whole problem on another tile, or on the build of the planned one
-  const Build &whole = fastest(c.m, c.n, c.k);
+  const Build &whole = fastest(c, c.m, c.n);
   if ((&whole != planned || !is_build(c, whole)) && grid_us(whole, c.m, c.n, c.k) < best_us) {
     best_us = grid_us(whole, c.m, c.n, c.k);
     best = {GridPart{on_build(c, whole, c.m, c.n)}};
@@ -194,7 +212,7 @@ std::vector<GridPart> split_grid(const tb_gemm_config &c) {
       continue;
     const int64_t m0 = rows ? cut : c.m, n0 = rows ? c.n : cut;
     const int64_t m1 = rows ? c.m - cut : c.m, n1 = rows ? c.n : c.n - cut;
-    const Build &rest = fastest(m1, n1, c.k);
+    const Build &rest = fastest(c, m1, n1);
     // 2 us for what a second launch leaves idle at its start and end
     const double us = over_build(c, *planned) * grid_us(*planned, m0, n0, c.k) +
                       grid_us(rest, m1, n1, c.k) + 2;

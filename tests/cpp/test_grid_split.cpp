@@ -20,10 +20,17 @@
 
 static int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// the hand-scheduled 256x256 kernel, where it adds the prior C in its loop
+static bool early_c(const tb_gemm_config &c) {
+  return c.block_m == 256 && c.block_n == 256 && c.block_k == 64 && c.wave_grid_m == 2 &&
+         c.wave_grid_n == 2 && c.stages == 2 && c.mfma == TB_MFMA_16X16X32 &&
+         c.k % 64 == 0 && c.k >= 18 * 64;
+}
+
 int main() {
   std::mt19937 rng(7);
   const int blocks[] = {64, 128, 192, 256};
-  int whole = 0, cut = 0;
+  int whole = 0, cut = 0, moved = 0;
   for (int i = 0; i < 20000; ++i) {
     tb_gemm_config c{};
     c.m = 1 + rng() % (1u << (4 + rng() % 13));
@@ -37,6 +44,14 @@ int main() {
     c.mapping = rng() % 5;
     c.group_m = 8;
     c.split_k = c.mapping == TB_MAP_SPLIT_K ? 4 : 1;
+    const bool accumulate = rng() % 2; // f32 C += A*B
+    c.c_dtype = accumulate ? TB_DTYPE_F32 : TB_DTYPE_F16;
+    c.acc_init = accumulate ? TB_ACC_INIT_LOAD_C : TB_ACC_INIT_ZERO;
+    if (rng() % 2)
+      c.k = (c.k + 63) / 64 * 64;
+    c.wave_grid_m = c.num_waves >= 4 ? 2 : 1;
+    c.wave_grid_n = c.num_waves / c.wave_grid_m;
+    c.mfma = rng() % 2 ? TB_MFMA_16X16X32 : TB_MFMA_32X32X16;
     const int64_t tiles = ceil_div(c.m, c.block_m) * ceil_div(c.n, c.block_n);
     const bool persistent =
         c.mapping == TB_MAP_PERSISTENT_TILE || c.mapping == TB_MAP_PERSISTENT_GROUPED;
@@ -60,6 +75,12 @@ int main() {
       CHECK(p.row0 % c.block_m == 0 && p.col0 % c.block_n == 0);
       CHECK(p.cfg.m > 0 && p.cfg.n > 0 && p.row0 + p.cfg.m <= c.m && p.col0 + p.cfg.n <= c.n);
       CHECK(p.cfg.k == c.k && p.cfg.split_k == 1 && p.cfg.n % 8 == 0);
+      CHECK(p.cfg.c_dtype == c.c_dtype && p.cfg.acc_init == c.acc_init);
+      // the kernel that adds the prior C inside its first k-tiles serves only
+      // plans that name it
+      if (accumulate && early_c(p.cfg))
+        CHECK(early_c(c));
+      moved += accumulate && p.cfg.block_m != c.block_m;
       const int64_t t = ceil_div(p.cfg.m, p.cfg.block_m) * ceil_div(p.cfg.n, p.cfg.block_n);
       const bool pers = p.cfg.mapping == TB_MAP_PERSISTENT_TILE ||
                         p.cfg.mapping == TB_MAP_PERSISTENT_GROUPED;
@@ -77,10 +98,11 @@ int main() {
     whole += parts.size() == 1;
     cut += parts.size() == 2;
   }
-  if (whole < 1000 || cut < 10) {
-    std::printf("FAILED: only %d whole and %d cut problems\n", whole, cut);
+  if (whole < 1000 || cut < 10 || moved < 500) {
+    std::printf("FAILED: only %d whole, %d cut and %d moved C += A*B problems\n", whole, cut,
+                moved);
     return 1;
   }
-  std::printf("ok: %d whole, %d cut\n", whole, cut);
+  std::printf("ok: %d whole, %d cut, %d moved\n", whole, cut, moved);
   return 0;
 }

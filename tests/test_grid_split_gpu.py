@@ -4,7 +4,8 @@ bit for bit with the planned kernel itself (a descriptor made from the plan's
 configuration runs exactly that): a whole problem on a finer tile, on a
 coarser one, rows and columns cut off as a second rectangle, ragged in M, N
 and K, with a bias row, an f32 C and persistent order; padding past the
-result is not written."""
+result is not written. f32 C += A*B has the planned kernel's bits too unless
+that one adds the prior C inside its loop; then its error is no larger."""
 import pytest
 import torch
 
@@ -26,7 +27,9 @@ CASES = [
     (512, 40000, 264, BIG, 2, {"bias": "f32"}),   # columns cut off
     (4200, 4200, 328, BIG, 2, {"persistent": True, "num_ctas": 256}),
     (4200, 4200, 328, BIG, 2, {"c_f32": True}),
-    (700, 1504, 2048, BIG, 2, {"c_f32": True}),
+    (700, 1504, 2048, BIG, 2, {"c_f32": True}),   # planned: prior C in the loop
+    (3072, 3072, 1280, MID, 3, {"c_f32": True}),  # large grids of small tiles
+    (2048, 2048, 2048, SMALL, 3, {"c_f32": True}),
     # split-K: 3 stages for 2, and 128x128 tiles on the 16x16x32 loop (splits of
     # unequal length, a partial last k-tile, fewer rows than a wave tile)
     (300, 520, 5000, (128, 64, 64), 2, {"split_k": 4, "bias": "f16"}),
@@ -66,9 +69,16 @@ def test_matches_planned_kernel(M, N, K, block, stages, options, device):
         got.append(c)
     if w.split_k > 1 and w.c_f32 and not w.module_attrs:
         assert torch.equal(got[0], got[1])  # fixed reduction order, C added first
-    if w.c_f32:
-        # the prior C is added before or after the products (atomic splits in
-        # any order): one rounding of each running sum apart
+    if w.c_f32 and w.split_k == 1:
+        in_loop = block == BIG and K % 64 == 0 and K >= 18 * 64
+        if not in_loop:  # the prior C is added last on both
+            assert torch.equal(got[0], got[1])
+        ref = a.double() @ b.double() + 3
+        err = [(c - ref).norm() for c in got]
+        assert err[0] <= err[1], err
+    elif w.c_f32:
+        # atomic splits are added in any order: one rounding of each running
+        # sum apart
         mag = a.float().abs() @ b.float().abs() + 3
         assert ((got[0] - got[1]).abs() <= (K + 2) * 2.0 ** -23 * mag).all()
         ref = a.double() @ b.double() + 3
