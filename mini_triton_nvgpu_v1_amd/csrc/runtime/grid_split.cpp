@@ -62,8 +62,12 @@ double round_us(const Build &b, int64_t tiles, double nk) {
   return b.c0 + nk * (b.lo + rise * (b.hi - b.lo));
 }
 
-double grid_us(const Build &b, int64_t m, int64_t n, int64_t k) {
-  const int64_t tiles = ceil_div(m, b.bm) * ceil_div(n, b.bn);
+int64_t tiles_of(int64_t m, int64_t n, int64_t bm, int64_t bn) {
+  return ceil_div(m, bm) * ceil_div(n, bn);
+}
+
+// A grid of `tiles` tiles that cost what b's do.
+double tiles_us(const Build &b, int64_t tiles, int64_t k) {
   const double nk = (double)ceil_div(k, 64);
   if (b.more > 0 && tiles > kCus) {
     const double rounds = (double)ceil_div(tiles, kCus);
@@ -73,7 +77,13 @@ double grid_us(const Build &b, int64_t m, int64_t n, int64_t k) {
   return (double)full * round_us(b, kCus, nk) + (rest ? round_us(b, rest, nk) : 0);
 }
 
-// The build of the planned tile's shape, or null.
+// An m x n problem on build b.
+double grid_us(const Build &b, int64_t m, int64_t n, int64_t k) {
+  return tiles_us(b, tiles_of(m, n, b.bm, b.bn), k);
+}
+
+// The build of the planned tile's shape or of its transpose, which costs the
+// same per tile; null: neither.
 const Build *build_of(const tb_gemm_config &c) {
   for (const Build &b : kBuilds)
     if ((b.bm == c.block_m && b.bn == c.block_n) ||
@@ -83,7 +93,8 @@ const Build *build_of(const tb_gemm_config &c) {
 }
 
 bool is_build(const tb_gemm_config &c, const Build &b) {
-  return c.block_k == 64 && c.stages == b.stages && c.num_waves == b.wgm * b.wgn;
+  return c.block_m == b.bm && c.block_n == b.bn && c.block_k == 64 && c.stages == b.stages &&
+         c.wave_grid_m == b.wgm && c.wave_grid_n == b.wgn && c.mfma == b.mfma;
 }
 
 // The time of the planned grid over its shape's build. A workgroup alone on
@@ -99,7 +110,7 @@ double over_build(const tb_gemm_config &c, const Build &b) {
     return 1;
   if (b.bm == 256 && b.bn == 256)
     return c.k >= 512 ? 1.15 : 1;
-  const int64_t tiles = ceil_div(c.m, c.block_m) * ceil_div(c.n, c.block_n);
+  const int64_t tiles = tiles_of(c.m, c.n, c.block_m, c.block_n);
   return tiles <= kCus && c.k >= 1024 && (c.stages == 2 || c.num_waves < 4) ? 1.2 : 1;
 }
 
@@ -121,7 +132,7 @@ bool adds_c_early(const Build &b, const tb_gemm_config &c) {
 // build may not worsen.
 const Build &fastest(const tb_gemm_config &c, int64_t m, int64_t n) {
   auto allowed = [&](const Build &b) {
-    return !adds_c_early(b, c) || (build_of(c) == &b && is_build(c, b));
+    return !adds_c_early(b, c) || is_build(c, b);
   };
   const Build *best = nullptr;
   double least = 0;
@@ -160,6 +171,11 @@ tb_gemm_config on_build(const tb_gemm_config &c, const Build &b, int64_t m, int6
 
 } // namespace
 
+double planned_us(const tb_gemm_config &c, int64_t m, int64_t n) {
+  const Build *b = build_of(c);
+  return b ? over_build(c, *b) * tiles_us(*b, tiles_of(m, n, c.block_m, c.block_n), c.k) : 0;
+}
+
 std::vector<GridPart> split_grid(const tb_gemm_config &c) {
   if (c.mapping == TB_MAP_SPLIT_K) {
     // The splits stay the plan's. Of workgroups alone on their CUs, 2 stages
@@ -190,15 +206,14 @@ std::vector<GridPart> split_grid(const tb_gemm_config &c) {
   // a persistent plan of fewer programs than CUs asks for a part of the chip
   if (persistent && c.num_programs < kCus)
     return {};
-  const Build *planned = build_of(c);
-  if (!planned)
+  if (!build_of(c))
     return {};
-  double best_us = 0.9 * over_build(c, *planned) * grid_us(*planned, c.m, c.n, c.k);
+  double best_us = 0.9 * planned_us(c, c.m, c.n);
   std::vector<GridPart> best;
 
   // the whole problem on another tile, or on the build of the planned one
   const Build &whole = fastest(c, c.m, c.n);
-  if ((&whole != planned || !is_build(c, whole)) && grid_us(whole, c.m, c.n, c.k) < best_us) {
+  if (!is_build(c, whole) && grid_us(whole, c.m, c.n, c.k) < best_us) {
     best_us = grid_us(whole, c.m, c.n, c.k);
     best = {GridPart{on_build(c, whole, c.m, c.n)}};
   }
@@ -214,8 +229,7 @@ std::vector<GridPart> split_grid(const tb_gemm_config &c) {
     const int64_t m1 = rows ? c.m - cut : c.m, n1 = rows ? c.n : c.n - cut;
     const Build &rest = fastest(c, m1, n1);
     // 2 us for what a second launch leaves idle at its start and end
-    const double us = over_build(c, *planned) * grid_us(*planned, m0, n0, c.k) +
-                      grid_us(rest, m1, n1, c.k) + 2;
+    const double us = planned_us(c, m0, n0) + grid_us(rest, m1, n1, c.k) + 2;
     if (us >= best_us)
       continue;
     best_us = us;

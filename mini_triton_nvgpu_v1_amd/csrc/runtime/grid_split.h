@@ -17,6 +17,10 @@ struct GridPart {
   int64_t row0 = 0, col0 = 0;
 };
 
+// Predicted time in us of an m x n rectangle of the problem on the planned
+// tile, in tile order (0: no estimate for that tile).
+double planned_us(const tb_gemm_config &c, int64_t m, int64_t n);
+
 // The rectangles a planned configuration runs as. Empty: as planned.
 std::vector<GridPart> split_grid(const tb_gemm_config &c);
 

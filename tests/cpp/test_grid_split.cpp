@@ -1,12 +1,14 @@
 // The rectangles a plan's launch runs (csrc/runtime/grid_split.h) tile C
 // exactly, on whole planned tiles, for random plans of every shape and order;
-// split-K plans keep their splits, and persistent plans of fewer programs than
-// CUs run as they are.
+// split-K plans keep their splits, persistent plans of fewer programs than CUs
+// run as they are, a plan and its transpose are predicted the same time, and
+// f32 C += A*B never moves to the kernel that adds the prior C in its loop.
 #include "runtime/grid_split.h"
 
 #include <cstdio>
 #include <cstdlib>
 #include <random>
+#include <utility>
 
 #define CHECK(x)                                                                            \
   do {                                                                                      \
@@ -25,6 +27,12 @@ static bool early_c(const tb_gemm_config &c) {
   return c.block_m == 256 && c.block_n == 256 && c.block_k == 64 && c.wave_grid_m == 2 &&
          c.wave_grid_n == 2 && c.stages == 2 && c.mfma == TB_MFMA_16X16X32 &&
          c.k % 64 == 0 && c.k >= 18 * 64;
+}
+
+static bool other_kernel(const tb_gemm_config &a, const tb_gemm_config &b) {
+  return a.block_m != b.block_m || a.block_n != b.block_n || a.block_k != b.block_k ||
+         a.stages != b.stages || a.wave_grid_m != b.wave_grid_m ||
+         a.wave_grid_n != b.wave_grid_n || a.mfma != b.mfma;
 }
 
 int main() {
@@ -51,12 +59,21 @@ int main() {
       c.k = (c.k + 63) / 64 * 64;
     c.wave_grid_m = c.num_waves >= 4 ? 2 : 1;
     c.wave_grid_n = c.num_waves / c.wave_grid_m;
-    c.mfma = rng() % 2 ? TB_MFMA_16X16X32 : TB_MFMA_32X32X16;
+    c.mfma = c.mapping != TB_MAP_SPLIT_K && rng() % 2 ? TB_MFMA_16X16X32 : TB_MFMA_32X32X16;
     const int64_t tiles = ceil_div(c.m, c.block_m) * ceil_div(c.n, c.block_n);
     const bool persistent =
         c.mapping == TB_MAP_PERSISTENT_TILE || c.mapping == TB_MAP_PERSISTENT_GROUPED;
     c.num_programs = persistent ? std::min<int64_t>(tiles, 1 + rng() % 512) : tiles * c.split_k;
     const std::vector<tbrt::GridPart> parts = tbrt::split_grid(c);
+    // the transposed problem on the transposed tile is the same grid
+    tb_gemm_config t = c;
+    std::swap(t.m, t.n);
+    std::swap(t.block_m, t.block_n);
+    std::swap(t.wave_grid_m, t.wave_grid_n);
+    CHECK(c.block_m == c.block_n || tbrt::planned_us(c, c.m, c.n) == tbrt::planned_us(t, t.m, t.n));
+    // one launch in place of the planned one is another kernel
+    if (parts.size() == 1)
+      CHECK(other_kernel(parts[0].cfg, c));
     if (persistent && c.num_programs < 256)
       CHECK(parts.empty());
     if (c.mapping == TB_MAP_SPLIT_K) { // as planned but for the stages
