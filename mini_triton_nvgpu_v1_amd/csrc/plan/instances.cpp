@@ -11,7 +11,7 @@
 namespace tb {
 
 static auto tie(const InstanceKey &k) {
-  return std::tie(k.bm, k.bn, k.bk, k.wgm, k.wgn, k.out, k.stages, k.epi, k.mfma);
+  return std::tie(k.bm, k.bn, k.bk, k.wgm, k.wgn, k.out, k.stages, k.epi, k.mfma, k.split);
 }
 bool InstanceKey::operator<(const InstanceKey &o) const { return tie(*this) < tie(o); }
 bool InstanceKey::operator==(const InstanceKey &o) const { return tie(*this) == tie(o); }
@@ -92,10 +92,11 @@ bool hasGfx950Instance(const InstanceKey &k) {
 
 std::string instanceName(const InstanceKey &k) {
   char buf[128];
-  snprintf(buf, sizeof buf, "tb_gemm_gfx950_%lldx%lldx%lld_w%lldx%lld_s%lld_out%d%s%s",
+  snprintf(buf, sizeof buf, "tb_gemm_gfx950_%lldx%lldx%lld_w%lldx%lld_s%lld_out%d%s%s%s",
            (long long)k.bm, (long long)k.bn, (long long)k.bk, (long long)k.wgm,
            (long long)k.wgn, (long long)k.stages, k.out,
-           k.mfma == TB_MFMA_16X16X32 ? "_16x16x32" : "", k.epi ? "_epi" : "");
+           k.mfma == TB_MFMA_16X16X32 ? "_16x16x32" : "", k.split ? "_split" : "",
+           k.epi ? "_epi" : "");
   return buf;
 }
 
@@ -111,6 +112,7 @@ InstanceKey instanceKeyOf(const tb_gemm_config &c) {
                         c.c_dtype == TB_DTYPE_F16, c.acc_init == TB_ACC_INIT_LOAD_C);
   k.epi = (c.epi_bias || c.epi_activation || c.epi_clamp) && c.mapping != TB_MAP_SPLIT_K;
   k.mfma = c.mfma;
+  k.split = c.mfma == TB_MFMA_16X16X32 && c.mapping == TB_MAP_SPLIT_K;
   return k;
 }
 
@@ -205,6 +207,9 @@ const ResourceRow kResources[] = {
 bool rowBinds(const ResourceRow &r, const InstanceKey &k, bool partialK) {
   const std::string f = r.family;
   const auto &a = r.args;
+  if (k.split)
+    return f == "gemm_mfma16g_split" && a.size() == 7 && a[0] == k.bm && a[1] == k.bn &&
+           a[2] == k.bk && a[3] == k.wgm && a[4] == k.wgn && a[5] == k.stages && a[6] == k.out;
   if (k.mfma == TB_MFMA_16X16X32) {
     // the hand-scheduled tile runs whole k-tiles; a partial last k-tile
     // runs the 16x16x32 loop's build of the same tile

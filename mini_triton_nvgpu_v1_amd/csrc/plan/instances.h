@@ -30,6 +30,8 @@ struct InstanceKey {
   int64_t stages = 0;
   int epi = 0;  // 1: the fused epilogue steps are compiled in
   int mfma = 0; // TB_MFMA_*
+  int split = 0; // 1: the split-K build of a 16x16x32 tile (a launch of a plan
+                 // may bind it; no plan names it and gfx950Instances() leaves it out)
   bool operator<(const InstanceKey &o) const;
   bool operator==(const InstanceKey &o) const;
 };

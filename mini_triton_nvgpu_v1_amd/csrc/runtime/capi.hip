@@ -169,24 +169,17 @@ int create_desc(const tb_gemm_config &c, tb_gemm_desc **out, bool part) {
   tbk::KernelKey key{(int)c.block_m, (int)c.block_n, (int)c.block_k,
                      (int)c.wave_grid_m, (int)c.wave_grid_n, out_mode,
                      (int)c.stages, epi, (int)c.mfma};
-  const bool split16 = c.mfma == TB_MFMA_16X16X32 && c.mapping == TB_MAP_SPLIT_K;
-  const tbk::KernelEntry *e = split16 ? tbk::find_split_kernel(key) : tbk::find_kernel(key);
+  const tb::InstanceKey ik = tb::instanceKeyOf(c);
+  const tbk::KernelEntry *e = ik.split ? tbk::find_split_kernel(key) : tbk::find_kernel(key);
   // an instance that spills to scratch is refused, as the plan refuses it
   // (the build-time table of the compiler's register report)
-  if (e && !split16) {
-    tb::InstanceKey ik;
-    ik.bm = c.block_m;
-    ik.bn = c.block_n;
-    ik.bk = c.block_k;
-    ik.wgm = c.wave_grid_m;
-    ik.wgn = c.wave_grid_n;
-    ik.out = out_mode;
-    ik.stages = c.stages;
-    ik.epi = epi;
-    ik.mfma = c.mfma;
+  if (e)
     if (const std::string why = tb::spillRefusal(ik, c.k % c.block_k != 0); !why.empty())
       return fail(why);
-  }
+  // a build that only launches of a plan bind is in no list a test goes
+  // through: it runs only if the table has it
+  if (e && part && !tb::instanceResources(ik, c.k % c.block_k != 0).known)
+    return fail(std::string("no compiler report for ") + e->name);
   if (!e) {
     char buf[256];
     snprintf(buf, sizeof buf,

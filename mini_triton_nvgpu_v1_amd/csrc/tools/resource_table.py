@@ -18,6 +18,7 @@ Kernel families and their template arguments (Itanium-mangled names):
   gemm_mfma16      EPI
   gemm_mfma16_f32  OUT EPI
   gemm_mfma16g     BM BN BK WGM WGN STAGES OUT EPI
+  gemm_mfma16g_split  BM BN BK WGM WGN STAGES OUT
 
 Usage: resource_table.py OUT.inc RES_FILE...
 """
@@ -27,7 +28,7 @@ import re
 import sys
 
 FAMILIES = ("gemm_kernel", "gemm_kernel_pw", "gemm_mfma16", "gemm_mfma16_f32",
-            "gemm_mfma16g")
+            "gemm_mfma16g", "gemm_mfma16g_split")
 NAME = re.compile(r"remark: Function Name: (\S+)")
 FIELD = re.compile(r"remark:\s+(TotalSGPRs|VGPRs|AGPRs|ScratchSize \[bytes/lane\]): (\d+)")
 MANGLED = re.compile(r"^_ZN3tbk(\d+)(\w+)$")
