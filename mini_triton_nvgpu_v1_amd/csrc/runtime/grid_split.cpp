@@ -125,30 +125,63 @@ bool adds_c_early(const Build &b, const tb_gemm_config &c) {
          c.k >= 18 * 64;
 }
 
-// The finest build within 5% of the fastest: what the constants leave out
-// (fused steps, an f32 C) is per element and spreads over more CUs
-// (1000 x 1496 x 712: 8.1 us predicted on 128x128, 7.7 on 64x128; 9.9 and
-// 8.3 measured). `c`: the plan, whose K it is and whose C += A*B rounding the
-// build may not worsen.
+// What the constants (f16 C, no fused steps) leave out of a grid, in us: the
+// prior C of C += A*B and its wider result, 6 bytes per element more at the
+// 4.9 TB/s of a copy (half as much again on the 256x256 tile, one wave per
+// SIMD: 4096^3 120 us against 97), and an activation, 5.9 us per round of
+// 256x256 tiles. Overlapped rounds hide some of both.
+double extra_us(const tb_gemm_config &c, const Build &b, int64_t m, int64_t n, int64_t tiles) {
+  const bool accumulate = c.acc_init == TB_ACC_INIT_LOAD_C;
+  double us = 0;
+  if (accumulate)
+    us += 6 * (double)m * (double)n / 4.9e6;
+  if (c.epi_activation != TB_ACT_NONE)
+    us += (double)ceil_div(tiles, kCus) * (double)(b.bm * b.bn) * 9e-5;
+  if (b.more > 0 && tiles > kCus)
+    return 0.6 * us;
+  return accumulate && b.bm == 256 && b.bn == 256 ? 1.6 * us : us;
+}
+
+// An m x n rectangle of plan c's problem on build b.
+double build_us(const tb_gemm_config &c, const Build &b, int64_t m, int64_t n) {
+  return grid_us(b, m, n, c.k) + extra_us(c, b, m, n, tiles_of(m, n, b.bm, b.bn));
+}
+
+// From a tile of which several fit a CU, a coarser one has to be predicted 25%
+// faster, not 10%: the constants know such grids to about 20% (231 x 7480 x
+// 552 on 64x64 in 2 stages: 7.7 us predicted and 8.0 measured, 6.8 and 10.8 on
+// 64x128). Of 424 random plans moved to a coarser tile with 10% for all and
+// no extra_us, 42 ran more than 5% longer than as planned, up to 1.35x.
+double margin(const tb_gemm_config &c, const Build &b) {
+  return b.bm * b.bn > c.block_m * c.block_n && build_of(c)->more > 0 ? 0.9 / 0.75 : 1;
+}
+
+// The finest build within 5% of the fastest: what the constants leave out is
+// per element and spreads over more CUs (1000 x 1496 x 712: 8.1 us predicted
+// on 128x128, 7.7 on 64x128; 9.9 and 8.3 measured). `c`: the plan, whose K it
+// is and whose C += A*B rounding the build may not worsen.
 const Build &fastest(const tb_gemm_config &c, int64_t m, int64_t n) {
+  auto us = [&](const Build &b) { return build_us(c, b, m, n) * margin(c, b); };
   auto allowed = [&](const Build &b) {
     return !adds_c_early(b, c) || is_build(c, b);
   };
   const Build *best = nullptr;
-  double least = 0;
   for (const Build &b : kBuilds)
-    if (allowed(b) && (!best || grid_us(b, m, n, c.k) < least)) {
+    if (allowed(b) && (!best || us(b) < us(*best)))
       best = &b;
-      least = grid_us(b, m, n, c.k);
-    }
+  const double least = us(*best);
   for (const Build &b : kBuilds) // coarse to fine
-    if (allowed(b) && grid_us(b, m, n, c.k) <= 1.05 * least)
+    if (allowed(b) && us(b) <= 1.05 * least)
       best = &b;
   return *best;
 }
 
 // The configuration of an m x n rectangle of c on build b: a plain grid in
-// grouped order, neighbours on one XCD once it fills the chip.
+// grouped order, neighbours on one XCD. Finer tiles re-read panels of A and B
+// more often than the planned ones, also in a grid of fewer tiles than CUs:
+// dealt over all XCDs, 71 x 14704 x 1920 took 25.4 us on 230 tiles of 64x128
+// where the planned 128x64 ones took 21.0, and 16.0 with neighbours together
+// (12 x 16104 x 1648 on 64x64 instead of 64x128: 16.4, 13.9 and 10.9).
 tb_gemm_config on_build(const tb_gemm_config &c, const Build &b, int64_t m, int64_t n) {
   tb_gemm_config r = c;
   r.m = m;
@@ -165,7 +198,7 @@ tb_gemm_config on_build(const tb_gemm_config &c, const Build &b, int64_t m, int6
   r.mapping = tm > 1 && tn > 1 ? TB_MAP_GROUPED_TILE : TB_MAP_TILE;
   r.group_m = r.mapping == TB_MAP_GROUPED_TILE ? 8 : 1;
   r.num_programs = tm * tn;
-  r.xcd_remap = tm * tn >= kCus ? 8 : 0;
+  r.xcd_remap = tm * tn >= 32 ? 8 : 0;
   return r;
 }
 
@@ -173,7 +206,10 @@ tb_gemm_config on_build(const tb_gemm_config &c, const Build &b, int64_t m, int6
 
 double planned_us(const tb_gemm_config &c, int64_t m, int64_t n) {
   const Build *b = build_of(c);
-  return b ? over_build(c, *b) * tiles_us(*b, tiles_of(m, n, c.block_m, c.block_n), c.k) : 0;
+  if (!b)
+    return 0;
+  const int64_t tiles = tiles_of(m, n, c.block_m, c.block_n);
+  return over_build(c, *b) * tiles_us(*b, tiles, c.k) + extra_us(c, *b, m, n, tiles);
 }
 
 std::vector<GridPart> split_grid(const tb_gemm_config &c) {
@@ -213,8 +249,9 @@ std::vector<GridPart> split_grid(const tb_gemm_config &c) {
 
   // the whole problem on another tile, or on the build of the planned one
   const Build &whole = fastest(c, c.m, c.n);
-  if (!is_build(c, whole) && grid_us(whole, c.m, c.n, c.k) < best_us) {
-    best_us = grid_us(whole, c.m, c.n, c.k);
+  const double whole_us = build_us(c, whole, c.m, c.n);
+  if (!is_build(c, whole) && whole_us * margin(c, whole) < best_us) {
+    best_us = whole_us;
     best = {GridPart{on_build(c, whole, c.m, c.n)}};
   }
   // the rows, or columns, of whole rounds as planned and the rest on the
@@ -229,7 +266,7 @@ std::vector<GridPart> split_grid(const tb_gemm_config &c) {
     const int64_t m1 = rows ? c.m - cut : c.m, n1 = rows ? c.n : c.n - cut;
     const Build &rest = fastest(c, m1, n1);
     // 2 us for what a second launch leaves idle at its start and end
-    const double us = planned_us(c, m0, n0) + grid_us(rest, m1, n1, c.k) + 2;
+    const double us = planned_us(c, m0, n0) + build_us(c, rest, m1, n1) + 2;
     if (us >= best_us)
       continue;
     best_us = us;
