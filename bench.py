@@ -124,7 +124,7 @@ def time_workload(w, steps: int, warmup: int, device, rounds: int = 5,
     ok = verify_output(w, A, B, C, bias, C0)
     return {"wall_s": statistics.median(walls), "avg_launch_ms": statistics.median(events),
             "round_wall_s": walls, "round_launch_ms": events, "round_clock_mhz": clocks,
-            "kernel": desc.kernel_name,
+            "kernel": desc.launched,  # what ran (a plan's launch may take another tile)
             "settle_launches": settle_launches, "verified": ok}
 
 

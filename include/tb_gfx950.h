@@ -163,6 +163,22 @@ int tb_plan_from_file(const char *path, tb_gemm_desc **out);
 int tb_desc_get_config(const tb_gemm_desc *desc, tb_gemm_config *out);
 /* Name of the selected kernel instance (valid while desc lives). */
 const char *tb_desc_kernel_name(const tb_gemm_desc *desc);
+/* One GEMM kernel launch of a descriptor (no reference counterpart: there a
+ * lowered kernel is what is launched). */
+typedef struct tb_launch_info {
+  const char *kernel_name; /* the instance that runs (a constant of the library) */
+  tb_gemm_config config;   /* its configuration; m and n: its rectangle of C */
+  int64_t row0, col0;      /* the rectangle's first row and column */
+  /* the s_waitcnt depths compiled into it (tb_kernel_waits) */
+  int32_t vmcnt_prologue, vmcnt_loop, lgkmcnt_loop;
+  /* its register report (tb_kernel_resources) */
+  int32_t vgprs, agprs, scratch_bytes;
+} tb_launch_info;
+/* How many GEMM kernels a launch of the descriptor runs (1, or 2 on two
+ * rectangles of C; a split-K reduction is not counted), and the i-th of them.
+ * For a descriptor made by tb_desc_create it is the descriptor's own kernel. */
+int tb_desc_launch_count(const tb_gemm_desc *desc);
+int tb_desc_launch_info(const tb_gemm_desc *desc, int i, tb_launch_info *out);
 /* Static LDS bytes per workgroup of the selected instance. */
 int64_t tb_desc_lds_bytes(const tb_gemm_desc *desc);
 

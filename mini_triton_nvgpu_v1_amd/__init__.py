@@ -17,7 +17,7 @@ import os
 import subprocess
 
 __all__ = [
-    "GemmConfig", "GemmDesc", "TbError", "lib", "build", "plan_from_mlir",
+    "GemmConfig", "GemmDesc", "LaunchInfo", "TbError", "lib", "build", "plan_from_mlir",
     "plan_from_file", "fill_seeded_f16", "kernel_names", "LIB_PATH", "TB_OPT",
     "DTYPE_F16", "DTYPE_F32", "ACC_INIT_ZERO", "ACC_INIT_LOAD_C", "MAP_TILE",
     "MAP_GROUPED_TILE", "MAP_SPLIT_K", "MAP_PERSISTENT_TILE",
@@ -78,6 +78,21 @@ class GemmConfig(ctypes.Structure):
         return f"GemmConfig({self.as_dict()})"
 
 
+class LaunchInfo(ctypes.Structure):
+    """Mirror of ``tb_launch_info``: one GEMM kernel launch of a descriptor."""
+    _fields_ = [
+        ("_kernel_name", ctypes.c_char_p), ("config", GemmConfig),
+        ("row0", ctypes.c_int64), ("col0", ctypes.c_int64),
+        ("vmcnt_prologue", ctypes.c_int32), ("vmcnt_loop", ctypes.c_int32),
+        ("lgkmcnt_loop", ctypes.c_int32), ("vgprs", ctypes.c_int32),
+        ("agprs", ctypes.c_int32), ("scratch_bytes", ctypes.c_int32),
+    ]
+
+    @property
+    def kernel_name(self) -> str:
+        return self._kernel_name.decode()
+
+
 _lib = None
 
 
@@ -122,6 +137,10 @@ def lib() -> ctypes.CDLL:
     L.tb_desc_get_config.restype = ctypes.c_int
     L.tb_desc_kernel_name.argtypes = [vp]
     L.tb_desc_kernel_name.restype = ctypes.c_char_p
+    L.tb_desc_launch_count.argtypes = [vp]
+    L.tb_desc_launch_count.restype = ctypes.c_int
+    L.tb_desc_launch_info.argtypes = [vp, ctypes.c_int, ctypes.POINTER(LaunchInfo)]
+    L.tb_desc_launch_info.restype = ctypes.c_int
     L.tb_desc_lds_bytes.argtypes = [vp]
     L.tb_desc_lds_bytes.restype = i64
     L.tb_workspace_bytes.argtypes = [vp]
@@ -261,6 +280,24 @@ class GemmDesc:
     @property
     def kernel_name(self) -> str:
         return lib().tb_desc_kernel_name(self._h).decode()
+
+    @property
+    def launches(self) -> list[LaunchInfo]:
+        """The GEMM kernels a launch runs, each with its rectangle of C
+        (config.m x config.n at row0, col0): the descriptor's own kernel, or
+        what a plan's launch runs in its place. Kernel names are read from the
+        library's memory: valid while the library is loaded."""
+        out = []
+        for i in range(lib().tb_desc_launch_count(self._h)):
+            info = LaunchInfo()
+            _check(lib().tb_desc_launch_info(self._h, i, ctypes.byref(info)))
+            out.append(info)
+        return out
+
+    @property
+    def launched(self) -> str:
+        """The names of the kernels a launch runs, joined by " + "."""
+        return " + ".join(x.kernel_name for x in self.launches)
 
     @property
     def lds_bytes(self) -> int:

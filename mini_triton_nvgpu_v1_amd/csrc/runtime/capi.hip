@@ -212,12 +212,23 @@ void choose_parts(tb_gemm_desc *d) {
   const std::string error = g_last_error; // a build that does not bind is no error here
   std::vector<tb_gemm_part> parts;
   for (const GridPart &g : split_grid(d->cfg)) {
-    tb_gemm_desc *sub = nullptr;
-    if (create_desc(g.cfg, &sub, true)) {
+    tb_gemm_desc *p = nullptr;
+    const int rc = create_desc(g.cfg, &p, true);
+    std::unique_ptr<tb_gemm_desc> sub(p);
+    // the waits compiled into the build are the ones its schedule states, as
+    // for the kernel a plan names
+    bool ok = rc == 0;
+    if (ok) {
+      const tb::InstanceSchedule s = tb::instanceSchedule(tb::instanceKeyOf(g.cfg));
+      int64_t have[3];
+      desc_waits(p, have);
+      ok = have[0] == s.vmPrologue && have[1] == s.vmLoop && have[2] == s.lgkmLoop;
+    }
+    if (!ok) {
       parts.clear();
       break;
     }
-    parts.push_back({std::unique_ptr<tb_gemm_desc>(sub), g.row0, g.col0});
+    parts.push_back({std::move(sub), g.row0, g.col0});
   }
   d->parts = std::move(parts);
   g_last_error = error;
@@ -413,6 +424,36 @@ int tb_desc_get_config(const tb_gemm_desc *desc, tb_gemm_config *out) {
 
 const char *tb_desc_kernel_name(const tb_gemm_desc *desc) {
   return desc && desc->entry ? desc->entry->name : "";
+}
+
+int tb_desc_launch_count(const tb_gemm_desc *desc) {
+  return !desc ? 0 : desc->parts.empty() ? 1 : (int)desc->parts.size();
+}
+
+int tb_desc_launch_info(const tb_gemm_desc *desc, int i, tb_launch_info *out) {
+  if (!desc || !out)
+    return fail("tb_desc_launch_info: NULL argument");
+  if (i < 0 || i >= tb_desc_launch_count(desc))
+    return fail("tb_desc_launch_info: no launch " + std::to_string(i));
+  const tb_gemm_desc *d = desc->parts.empty() ? desc : desc->parts[i].desc.get();
+  *out = {};
+  out->kernel_name = d->entry->name;
+  out->config = d->cfg;
+  if (!desc->parts.empty()) {
+    out->row0 = desc->parts[i].row0;
+    out->col0 = desc->parts[i].col0;
+  }
+  out->vmcnt_prologue = d->entry->vm_prologue;
+  out->vmcnt_loop = d->entry->vm_loop;
+  out->lgkmcnt_loop = d->entry->lgkm_loop;
+  const tb::InstanceResources r =
+      tb::instanceResources(tb::instanceKeyOf(d->cfg), d->cfg.k % d->cfg.block_k != 0);
+  if (!r.known)
+    return fail(std::string("tb_desc_launch_info: no compiler report for ") + d->entry->name);
+  out->vgprs = (int32_t)r.vgprs;
+  out->agprs = (int32_t)r.agprs;
+  out->scratch_bytes = (int32_t)r.scratchBytes;
+  return 0;
 }
 
 int64_t tb_desc_lds_bytes(const tb_gemm_desc *desc) {

@@ -548,7 +548,8 @@ def main(argv=None) -> int:
             "gpu_state_after_case": query_gpu_state(),
             "case_preheat": case_preheat,
             "verify": check,
-            "mini": {"kernel": runner.desc.kernel_name,
+            "mini": {"kernel": runner.desc.launched,  # what ran
+                     "planned_kernel": runner.desc.kernel_name,
                      "plan_pipeline_ms": round(runner.plan_ms, 3),
                      "summary_ns": ms, "summary_gflops": mg, "samples": mini},
             "other": None if os_ is None else {

@@ -71,7 +71,7 @@ def main() -> int:
     for _ in range(args.reps):
         desc.launch(A, B, C, ws, stream=stream, bias=bias)
     torch.cuda.synchronize()
-    print(f"profiling: {args.reps} launches of {desc.kernel_name} ({w.name})", flush=True)
+    print(f"profiling: {args.reps} launches of {desc.launched} ({w.name})", flush=True)
     if args.hipblaslt and not w.c_f32:
         # the vendor library on the same operands, for side-by-side counters
         for _ in range(args.reps):

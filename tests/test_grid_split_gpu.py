@@ -16,40 +16,59 @@ pytestmark = pytest.mark.gpu
 
 ATOMIC = {"tb.reduction-mode": '"split_k_parallel"'}
 BIG, MID, SMALL = (256, 256, 64), (128, 128, 64), (64, 64, 64)
-# (M, N, K, block, stages, options)
+T256, T256x128, T128 = ("256x256x64_w2x2_s2_out{}_16x16x32", "256x128x64_w4x2_s3_out{}_16x16x32",
+                        "128x128x64_w2x2_s3_out{}_16x16x32")
+T64x128, T64 = "64x128x64_w2x4_s3_out{}", "64x64x64_w2x2_s3_out{}"
+SPLIT = "128x128x64_w2x2_s3_out{}_16x16x32_split"
+# (M, N, K, block, stages, options, the kernels that run with their first row
+# and column)
 CASES = [
-    (1, 8, 8, MID, 3, {}),                        # one element row, K below a k-tile
-    (129, 136, 72, MID, 2, {"bias": "f16", "activation": "silu"}),
-    (1000, 1496, 712, BIG, 2, {"bias": "f32", "clamp_min": -0.5, "clamp_max": 0.5}),
-    (900, 1032, 1032, MID, 2, {}),                # 2-stage plan with a long K
-    (2048, 2056, 200, SMALL, 2, {}),              # a coarser tile
-    (4104, 4096, 520, BIG, 2, {"bias": "f16"}),   # 8 rows past a whole round
-    (512, 40000, 264, BIG, 2, {"bias": "f32"}),   # columns cut off
-    (4200, 4200, 328, BIG, 2, {"persistent": True, "num_ctas": 256}),
-    (4200, 4200, 328, BIG, 2, {"c_f32": True}),
-    (700, 1504, 2048, BIG, 2, {"c_f32": True}),   # planned: prior C in the loop
-    (3072, 3072, 1280, MID, 3, {"c_f32": True}),  # large grids of small tiles
-    (2048, 2048, 2048, SMALL, 3, {"c_f32": True}),
+    # one element row, K below a k-tile
+    (1, 8, 8, MID, 3, {}, [(T64, 0, 0)]),
+    (129, 136, 72, MID, 2, {"bias": "f16", "activation": "silu"}, [(T64 + "_epi", 0, 0)]),
+    (1000, 1496, 712, BIG, 2, {"bias": "f32", "clamp_min": -0.5, "clamp_max": 0.5},
+     [(T64x128 + "_epi", 0, 0)]),
+    (900, 1032, 1032, MID, 2, {}, [(T64, 0, 0)]),  # 2-stage plan with a long K
+    (2048, 2056, 200, SMALL, 2, {}, [(T256x128, 0, 0)]),  # a coarser tile
+    (4104, 4096, 520, BIG, 2, {"bias": "f16"},    # 8 rows past a whole round
+     [(T256 + "_epi", 0, 0), (T64 + "_epi", 4096, 0)]),
+    (512, 40000, 264, BIG, 2, {"bias": "f32"},    # columns cut off
+     [(T256 + "_epi", 0, 0), (T128 + "_epi", 0, 32768)]),
+    (4200, 4200, 328, BIG, 2, {"persistent": True, "num_ctas": 256},
+     [(T256, 0, 0), (T64x128, 3840, 0)]),
+    (4200, 4200, 328, BIG, 2, {"c_f32": True}, [(T64x128, 0, 0)]),
+    (4104, 4096, 2056, BIG, 2, {"c_f32": True}, [(T256, 0, 0), (T64, 4096, 0)]),
+    (700, 1504, 2048, BIG, 2, {"c_f32": True}, [(T64x128, 0, 0)]),  # planned: C in the loop
+    (3072, 3072, 1280, MID, 3, {"c_f32": True}, [(T128, 0, 0)]),  # not to 256x256
+    (2560, 2560, 1280, MID, 3, {"c_f32": True}, [(T256x128, 0, 0)]),
+    (2048, 2048, 2048, SMALL, 3, {"c_f32": True}, [(T128, 0, 0)]),
     # split-K: 3 stages for 2, and 128x128 tiles on the 16x16x32 loop (splits of
     # unequal length, a partial last k-tile, fewer rows than a wave tile)
-    (300, 520, 5000, (128, 64, 64), 2, {"split_k": 4, "bias": "f16"}),
-    (300, 520, 5000, MID, 2, {"split_k": 4, "bias": "f16", "activation": "relu"}),
-    (129, 136, 9224, MID, 3, {"split_k": 16}),
-    (7, 1032, 4096, MID, 2, {"split_k": 7, "c_f32": True}),
-    (1000, 776, 4168, MID, 2, {"split_k": 4, "c_f32": True, "module_attrs": ATOMIC}),
-    (129, 8, 9000, MID, 4, {"split_k": 3, "c_f32": True, "module_attrs": ATOMIC}),
+    (300, 520, 5000, (128, 64, 64), 2, {"split_k": 4, "bias": "f16"},
+     [("128x64x64_w4x1_s3_out1", 0, 0)]),
+    (300, 520, 5000, MID, 2, {"split_k": 4, "bias": "f16", "activation": "relu"},
+     [(SPLIT, 0, 0)]),
+    (129, 136, 9224, MID, 3, {"split_k": 16}, [(SPLIT, 0, 0)]),
+    (7, 1032, 4096, MID, 2, {"split_k": 7, "c_f32": True}, [(SPLIT, 0, 0)]),
+    (1000, 776, 4168, MID, 2, {"split_k": 4, "c_f32": True, "module_attrs": ATOMIC},
+     [(SPLIT, 0, 0)]),
+    (129, 8, 9000, MID, 4, {"split_k": 3, "c_f32": True, "module_attrs": ATOMIC},
+     [(SPLIT, 0, 0)]),
 ]
 
 
-@pytest.mark.parametrize("M,N,K,block,stages,options", CASES,
+@pytest.mark.parametrize("M,N,K,block,stages,options,runs", CASES,
                          ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else None)
-def test_matches_planned_kernel(M, N, K, block, stages, options, device):
+def test_matches_planned_kernel(M, N, K, block, stages, options, runs, device):
     print(f"grid split {M}x{N}x{K} {block} {options}", flush=True)
     w = configs.Workload("w", M, N, K, 0, configs.NORMAL, block, num_waves=4, stages=stages,
                          exact_tile=False, **options)
     plan = tb.plan_from_mlir(w.mlir())
     exact = tb.GemmDesc.from_config(plan.config)
-    assert exact.kernel_name == plan.kernel_name
+    assert exact.launched == exact.kernel_name == plan.kernel_name
+    out = int(plan.kernel_name.split("_out")[1][0])
+    assert ([(x.kernel_name, x.row0, x.col0) for x in plan.launches]
+            == [("tb_gemm_gfx950_" + name.format(out), r, c) for name, r, c in runs])
     g = torch.Generator(device=device).manual_seed(M + N + K)
     a = torch.randn(M, K, generator=g, device=device).half()
     b = (torch.randn(K, N, generator=g, device=device) / K ** 0.5).half()
@@ -94,6 +113,7 @@ def test_two_rectangles_in_a_graph(device):
     print(f"grid split graph {M}x{N}x{K}", flush=True)
     w = configs.Workload("w", M, N, K, 0, configs.NORMAL, BIG, num_waves=4, exact_tile=False)
     desc = tb.plan_from_mlir(w.mlir())
+    assert len(desc.launches) == 2
     a = torch.randn(M, K, device=device).half()
     b = (torch.randn(K, N, device=device) / K ** 0.5).half()
     c = torch.empty(M, N, device=device, dtype=torch.float16)
