@@ -21,6 +21,7 @@ import torch
 import mini_triton_nvgpu_v1_amd as tb
 import oracle
 from mini_triton_nvgpu_v1_amd import configs
+from test_gemm_gpu import kernels_of
 
 pytestmark = pytest.mark.gpu
 RTOL = 1e-2
@@ -57,7 +58,7 @@ def _run_and_check(desc, w, A, B, device, c0=None, c_dtype=torch.float16):
     oracle.epilogue_f64(ref, bias_ref, ACT[w.activation], _clamp_bits(w),
                         w.clamp_min or 0.0, w.clamp_max or 0.0)
     bad, err, worst = oracle.check_tolerance(got, ref, rtol=RTOL)
-    print(f"{w.name} via {desc.kernel_name}: violations={bad} max|err|={err:.3e}",
+    print(f"{w.name} via {desc.launched}: violations={bad} max|err|={err:.3e}",
           flush=True)
     assert bad == 0, f"{bad} elements outside tolerance; worst {err} at {worst}"
     return got, ref
@@ -95,7 +96,8 @@ def test_fused_epilogue_f16(w, device):
     desc = tb.plan_from_mlir(w.mlir())
     assert desc.config == w.direct_config()
     A, B = oracle.config_inputs(w.M, w.N, w.K, w.seed, w.dist)
-    _run_and_check(desc, w, A, B, device)
+    for d in kernels_of(desc):  # what the launch runs, and the planned kernel
+        _run_and_check(d, w, A, B, device)
 
 
 def test_fused_epilogue_f32_accumulate(device):
@@ -109,7 +111,8 @@ def test_fused_epilogue_f32_accumulate(device):
     assert "_out2" in desc.kernel_name and desc.kernel_name.endswith("_epi")
     A, B = oracle.config_inputs(w.M, w.N, w.K, w.seed, w.dist)
     C0 = oracle.fill_f16(w.M, w.N, 0x5EED0601, oracle.UNIFORM, 2.0).astype(np.float32)
-    _run_and_check(desc, w, A, B, device, c0=C0, c_dtype=torch.float32)
+    for d in kernels_of(desc):
+        _run_and_check(d, w, A, B, device, c0=C0, c_dtype=torch.float32)
 
 
 def test_fused_epilogue_f32_plain_store(device):

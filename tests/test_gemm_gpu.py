@@ -42,6 +42,14 @@ def run_desc(desc: tb.GemmDesc, A16, B16, device, c_init=None, c_dtype=torch.flo
     return dC.cpu().numpy()
 
 
+def kernels_of(desc):
+    """The plan's descriptor and, where its launch runs another tile or two
+    rectangles, the planned kernel itself."""
+    yield desc
+    if desc.launched != desc.kernel_name:
+        yield tb.GemmDesc.from_config(desc.config)
+
+
 def check(got, A16, B16, init=None, rows=None):
     """Full check, or a list of (row_begin, row_end) blocks."""
     blocks = rows or [(0, A16.shape[0])]
@@ -59,9 +67,8 @@ def test_workload_parity(w, device):
     """The product path: tb.matmul module text -> plan pipeline -> kernel."""
     print(f"workload {w.name} {w.M}x{w.N}x{w.K}", flush=True)
     A, B = oracle.config_inputs(w.M, w.N, w.K, w.seed, w.dist)
-    desc = tb.plan_from_mlir(w.mlir())
-    got = run_desc(desc, A, B, device)
-    check(got, A, B)
+    for desc in kernels_of(tb.plan_from_mlir(w.mlir())):
+        check(run_desc(desc, A, B, device), A, B)
 
 
 @pytest.fixture(scope="module")
@@ -165,8 +172,9 @@ def test_plan_module_f32_accumulate(name, M, N, K, tile, warps, extra, device):
     assert desc.config.acc_init == tb.ACC_INIT_LOAD_C
     A, B = oracle.config_inputs(M, N, K, 0x5EED0500, oracle.UNIFORM)
     C0 = oracle.fill_f16(M, N, 0x5EED0501, oracle.UNIFORM, 4.0).astype(np.float32)
-    got = run_desc(desc, A, B, device, c_init=C0.copy(), c_dtype=torch.float32)
-    check(got, A, B, init=C0)
+    for d in kernels_of(desc):
+        got = run_desc(d, A, B, device, c_init=C0.copy(), c_dtype=torch.float32)
+        check(got, A, B, init=C0)
 
 
 # Large shapes with edges in M, N and K, through the plan pipeline: partial
@@ -202,8 +210,8 @@ def test_large_ragged_parity(w, device):
     # the 16x16x32 instance takes the 256x256x64 4-wave tiles, ragged M, N
     # and K included
     assert ("16x16x32" in desc.kernel_name) == w.mfma16_supported(), desc.kernel_name
-    got = run_desc(desc, A, B, device)
-    check(got, A, B)
+    for d in kernels_of(desc):
+        check(run_desc(d, A, B, device), A, B)
 
 
 RAGGED_SHAPES = [(1, 8, 8), (33, 24, 16), (97, 88, 40), (200, 136, 72),

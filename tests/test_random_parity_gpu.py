@@ -18,7 +18,7 @@ import torch
 
 import mini_triton_nvgpu_v1_amd as tb
 import oracle
-from test_gemm_gpu import _every_instance, _spills, run_desc
+from test_gemm_gpu import _every_instance, _spills, kernels_of, run_desc
 
 pytestmark = pytest.mark.gpu
 RTOL = 1e-2
@@ -212,14 +212,15 @@ def test_random_plan_pipeline_parity(device):
             continue
         print(f"plan case {case}: {M}x{N}x{K} tile {(bm, bn, bk)} waves {w.num_waves} "
               f"stages {w.stages} split {split} persistent {persistent} -> "
-              f"{desc.kernel_name}", flush=True)
+              f"{desc.kernel_name}, runs {desc.launched}", flush=True)
         A, B = oracle.config_inputs(M, N, K, w.seed, w.dist)
-        got = run_desc(desc, A, B, device)
         ref = oracle.gemm_f64(A, B)
-        bad, err, worst = oracle.check_tolerance(got, ref, rtol=RTOL)
         ran += 1
-        if bad:
-            failures.append(f"plan case {case} ({desc.kernel_name}): {bad} violations, "
-                            f"worst {err} at {worst}")
+        for d in kernels_of(desc):  # what the launch runs, and the planned kernel
+            got = run_desc(d, A, B, device)
+            bad, err, worst = oracle.check_tolerance(got, ref, rtol=RTOL)
+            if bad:
+                failures.append(f"plan case {case} ({d.launched}): {bad} violations, "
+                                f"worst {err} at {worst}")
     assert not failures, "\n".join(failures)
     assert ran >= PLAN_CASES // 2, f"only {ran} of {PLAN_CASES} modules planned"
