@@ -7,10 +7,10 @@
 // took two rounds, the second a quarter full, 178 us. C does not depend on
 // the tile: every build adds the products of an element in the same k order
 // in f32 (bit-identical for f16 and plain f32 results; for f32 C += A*B see
-// adds_c_early). So the launch of a plan may
-// run the same problem on another tile, or cut it in two rectangles: the rows
-// (or columns) that fill whole rounds on the planned tile, and the rest on a
-// tile that spreads it over the chip.
+// adds_c_early). So the launch of a plan may run the same problem on another
+// tile, or cut it in two rectangles: the rows (or columns) that fill whole
+// rounds on the planned tile, and the rest on a tile that spreads it over the
+// chip.
 //
 // The choice is by time, from two measured constants per tile: a grid's
 // round of up to 256 tiles takes c0 + (K / 64) * c1(fill) us, where c1 rises
@@ -127,9 +127,10 @@ bool adds_c_early(const Build &b, const tb_gemm_config &c) {
 
 // What the constants (f16 C, no fused steps) leave out of a grid, in us: the
 // prior C of C += A*B and its wider result, 6 bytes per element more at the
-// 4.9 TB/s of a copy (half as much again on the 256x256 tile, one wave per
-// SIMD: 4096^3 120 us against 97), and an activation, 5.9 us per round of
-// 256x256 tiles. Overlapped rounds hide some of both.
+// 4.9 TB/s of a copy, and an activation, 5.9 us per round of 256x256 tiles; 1.6
+// times both for C += A*B on the 256x256 tile, whose lone wave per SIMD does
+// nothing else meanwhile (2841 x 2936 x 384 with GELU: 13.3 us predicted
+// without, 34.4 measured). Overlapped rounds hide some of it.
 double extra_us(const tb_gemm_config &c, const Build &b, int64_t m, int64_t n, int64_t tiles) {
   const bool accumulate = c.acc_init == TB_ACC_INIT_LOAD_C;
   double us = 0;
