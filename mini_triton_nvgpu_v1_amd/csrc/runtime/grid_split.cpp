@@ -26,16 +26,17 @@
 // overlap: each costs 2.2 and 0.92 us and the K part 0.3 and 0.195 us per 64
 // of K and round (1024 tiles, K = 64 / 1024 / 4096: 12.0 / 27.0 / 88.2 us on
 // 64x128, 7.0 / 17.6 / 55.3 on 64x64).
-// A choice has to be predicted 10% faster than the plan as it stands: the
-// constants reproduce the measured times to about 8%.
+// A choice has to save 10% of the planned grid's time by these constants, which
+// reproduce the measured times to about 8%.
 #include "grid_split.h"
 
 #include <algorithm>
+#include <bitset>
 
 namespace tbrt {
 namespace {
 
-constexpr int64_t kCus = 256;
+constexpr int64_t kCus = 256, kXcds = 8;
 
 // A tile the launch may choose: its build, and its cost per round.
 struct Build {
@@ -127,25 +128,19 @@ bool adds_c_early(const Build &b, const tb_gemm_config &c) {
 
 // What the constants (f16 C, no fused steps) leave out of a grid, in us: the
 // prior C of C += A*B and its wider result, 6 bytes per element more at the
-// 4.9 TB/s of a copy, and an activation, 5.9 us per round of 256x256 tiles; 1.6
-// times both for C += A*B on the 256x256 tile, whose lone wave per SIMD does
-// nothing else meanwhile (2841 x 2936 x 384 with GELU: 13.3 us predicted
-// without, 34.4 measured). Overlapped rounds hide some of it.
+// 4.9 TB/s of a copy, and an activation, 5.9 us per round of 256x256 tiles
+// (ReLU 1.6), twice that in a C += A*B, which dispatches it per 16-row block.
+// Overlapped rounds hide some of it. Without this, 3609 x 4400 x 192, C += A*B
+// on 64x128, moved to 256x128: 25.4 -> 34.0 us.
 double extra_us(const tb_gemm_config &c, const Build &b, int64_t m, int64_t n, int64_t tiles) {
   const bool accumulate = c.acc_init == TB_ACC_INIT_LOAD_C;
   double us = 0;
   if (accumulate)
     us += 6 * (double)m * (double)n / 4.9e6;
   if (c.epi_activation != TB_ACT_NONE)
-    us += (double)ceil_div(tiles, kCus) * (double)(b.bm * b.bn) * 9e-5;
-  if (b.more > 0 && tiles > kCus)
-    return 0.6 * us;
-  return accumulate && b.bm == 256 && b.bn == 256 ? 1.6 * us : us;
-}
-
-// An m x n rectangle of plan c's problem on build b.
-double build_us(const tb_gemm_config &c, const Build &b, int64_t m, int64_t n) {
-  return grid_us(b, m, n, c.k) + extra_us(c, b, m, n, tiles_of(m, n, b.bm, b.bn));
+    us += (double)ceil_div(tiles, kCus) * (double)(b.bm * b.bn) *
+          (c.epi_activation == TB_ACT_RELU ? 2.5e-5 : 9e-5) * (accumulate ? 2 : 1);
+  return b.more > 0 && tiles > kCus ? 0.6 * us : us;
 }
 
 // From a tile of which several fit a CU, a coarser one has to be predicted 25%
@@ -157,12 +152,18 @@ double margin(const tb_gemm_config &c, const Build &b) {
   return b.bm * b.bn > c.block_m * c.block_n && build_of(c)->more > 0 ? 0.9 / 0.75 : 1;
 }
 
+// An m x n rectangle of plan c's problem on build b, as a candidate.
+double build_us(const tb_gemm_config &c, const Build &b, int64_t m, int64_t n) {
+  return grid_us(b, m, n, c.k) * margin(c, b) +
+         extra_us(c, b, m, n, tiles_of(m, n, b.bm, b.bn));
+}
+
 // The finest build within 5% of the fastest: what the constants leave out is
 // per element and spreads over more CUs (1000 x 1496 x 712: 8.1 us predicted
 // on 128x128, 7.7 on 64x128; 9.9 and 8.3 measured). `c`: the plan, whose K it
 // is and whose C += A*B rounding the build may not worsen.
 const Build &fastest(const tb_gemm_config &c, int64_t m, int64_t n) {
-  auto us = [&](const Build &b) { return build_us(c, b, m, n) * margin(c, b); };
+  auto us = [&](const Build &b) { return build_us(c, b, m, n); };
   auto allowed = [&](const Build &b) {
     return !adds_c_early(b, c) || is_build(c, b);
   };
@@ -177,12 +178,45 @@ const Build &fastest(const tb_gemm_config &c, int64_t m, int64_t n) {
   return *best;
 }
 
+// Rows and columns of C (as rows of A, columns of B) that the XCDs of a grid
+// of at most 256 tiles read together, in grouped order by eights: blocks are
+// dealt to the XCDs in turn, and with `remap` each XCD takes a contiguous run
+// of programs (program_of_block and map_program of the kernels).
+int64_t xcd_lines(int64_t tm, int64_t tn, int64_t bm, int64_t bn, bool remap) {
+  const int64_t nprog = tm * tn, gm = tm > 1 && tn > 1 ? 8 : 1;
+  int64_t lines = 0;
+  for (int64_t x = 0; x < kXcds; ++x) {
+    std::bitset<kCus> rows, cols;
+    for (int64_t block = x; block < nprog; block += kXcds) {
+      const int64_t pid =
+          remap ? x * (nprog / kXcds) + std::min(x, nprog % kXcds) + block / kXcds : block;
+      const int64_t first = pid / (gm * tn) * gm, in_group = pid % (gm * tn);
+      const int64_t gsz = std::min(tm - first, gm);
+      rows.set((size_t)(first + in_group % gsz));
+      cols.set((size_t)(in_group / gsz));
+    }
+    lines += (int64_t)rows.count() * bm + (int64_t)cols.count() * bn;
+  }
+  return lines;
+}
+
+// Whether neighbours of a grid run on one XCD: where that order has the XCDs
+// read a quarter less of A and B from memory (218 x 2968 x 2456 on 64x64: 19.8 ->
+// 16.2 us; 314 x 3032 x 568: 8.7 -> 7.8; from 80% on the other order was as
+// fast or up to 4% faster), or where a single row of tiles shares the cache
+// lines of B's rows (41 x 12904 x 1464 on 64x64: 15.1 -> 9.5). A short K (272 to
+// 470) gained nothing, a full chip always does.
+bool neighbours_on_one_xcd(int64_t tm, int64_t tn, int64_t k, int64_t bm, int64_t bn) {
+  if (tm * tn >= kCus)
+    return true;
+  if (tm * tn < 32 || k < 512)
+    return false;
+  return tm == 1 ||
+         4 * xcd_lines(tm, tn, bm, bn, true) <= 3 * xcd_lines(tm, tn, bm, bn, false);
+}
+
 // The configuration of an m x n rectangle of c on build b: a plain grid in
-// grouped order, neighbours on one XCD. Finer tiles re-read panels of A and B
-// more often than the planned ones, also in a grid of fewer tiles than CUs:
-// dealt over all XCDs, 71 x 14704 x 1920 took 25.4 us on 230 tiles of 64x128
-// where the planned 128x64 ones took 21.0, and 16.0 with neighbours together
-// (12 x 16104 x 1648 on 64x64 instead of 64x128: 16.4, 13.9 and 10.9).
+// grouped order.
 tb_gemm_config on_build(const tb_gemm_config &c, const Build &b, int64_t m, int64_t n) {
   tb_gemm_config r = c;
   r.m = m;
@@ -199,18 +233,18 @@ tb_gemm_config on_build(const tb_gemm_config &c, const Build &b, int64_t m, int6
   r.mapping = tm > 1 && tn > 1 ? TB_MAP_GROUPED_TILE : TB_MAP_TILE;
   r.group_m = r.mapping == TB_MAP_GROUPED_TILE ? 8 : 1;
   r.num_programs = tm * tn;
-  r.xcd_remap = tm * tn >= 32 ? 8 : 0;
+  r.xcd_remap = neighbours_on_one_xcd(tm, tn, c.k, b.bm, b.bn) ? kXcds : 0;
   return r;
 }
 
 } // namespace
 
-double planned_us(const tb_gemm_config &c, int64_t m, int64_t n) {
+double planned_us(const tb_gemm_config &c, int64_t m, int64_t n, double share) {
   const Build *b = build_of(c);
   if (!b)
     return 0;
   const int64_t tiles = tiles_of(m, n, c.block_m, c.block_n);
-  return over_build(c, *b) * tiles_us(*b, tiles, c.k) + extra_us(c, *b, m, n, tiles);
+  return share * over_build(c, *b) * tiles_us(*b, tiles, c.k) + extra_us(c, *b, m, n, tiles);
 }
 
 std::vector<GridPart> split_grid(const tb_gemm_config &c) {
@@ -245,13 +279,13 @@ std::vector<GridPart> split_grid(const tb_gemm_config &c) {
     return {};
   if (!build_of(c))
     return {};
-  double best_us = 0.9 * planned_us(c, c.m, c.n);
+  double best_us = planned_us(c, c.m, c.n, 0.9);
   std::vector<GridPart> best;
 
   // the whole problem on another tile, or on the build of the planned one
   const Build &whole = fastest(c, c.m, c.n);
   const double whole_us = build_us(c, whole, c.m, c.n);
-  if (!is_build(c, whole) && whole_us * margin(c, whole) < best_us) {
+  if (!is_build(c, whole) && whole_us < best_us) {
     best_us = whole_us;
     best = {GridPart{on_build(c, whole, c.m, c.n)}};
   }

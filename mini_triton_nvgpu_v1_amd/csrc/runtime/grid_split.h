@@ -18,8 +18,9 @@ struct GridPart {
 };
 
 // Predicted time in us of an m x n rectangle of the problem on the planned
-// tile, in tile order (0: no estimate for that tile).
-double planned_us(const tb_gemm_config &c, int64_t m, int64_t n);
+// tile (0: no estimate for that tile), `share` of the part that depends on
+// the tile.
+double planned_us(const tb_gemm_config &c, int64_t m, int64_t n, double share = 1);
 
 // The rectangles a planned configuration runs as. Empty: as planned.
 std::vector<GridPart> split_grid(const tb_gemm_config &c);

@@ -36,7 +36,7 @@ CASES = [
      [(T256 + "_epi", 0, 0), (T128 + "_epi", 0, 32768)]),
     (4200, 4200, 328, BIG, 2, {"persistent": True, "num_ctas": 256},
      [(T256, 0, 0), (T64x128, 3840, 0)]),
-    (4200, 4200, 328, BIG, 2, {"c_f32": True}, [(T64x128, 0, 0)]),
+    (4200, 4200, 328, BIG, 2, {"c_f32": True}, [(T256, 0, 0), (T64, 3840, 0)]),
     (4104, 4096, 2056, BIG, 2, {"c_f32": True}, [(T256, 0, 0), (T64, 4096, 0)]),
     (700, 1504, 2048, BIG, 2, {"c_f32": True}, [(T64x128, 0, 0)]),  # planned: C in the loop
     (3072, 3072, 1280, MID, 3, {"c_f32": True}, [(T128, 0, 0)]),  # not to 256x256
