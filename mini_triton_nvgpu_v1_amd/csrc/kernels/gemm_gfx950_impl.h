@@ -1564,6 +1564,36 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_kernel(GemmParams p) {
           }
           asm volatile("" ::: "memory");
           if constexpr (OUT == kOutF32Atomic) {
+            // One wave of 64 columns or fewer, in up to 8 workgroups: nearly
+            // nobody to share the lines with, so the wave's own reads and
+            // address arithmetic are what it waits for, and four columns a
+            // lane take one read and one offset. 64x64x32, against whole
+            // lines: 64^3 in 2 splits 3.7-4.2 us and 5.2 (3.55 and 4.71 per
+            // kernel), 128^2 in 2 (8 workgroups) 4.3 and 4.9, 64^2 in 8 5.4
+            // and 5.9. With more the lines win: 64^2 in 16 5.9 and 5.5, 128^2
+            // in 8 (32) 6.8 and 6.1. Two waves lose from 4 workgroups on or
+            // sooner; a wave of 128 columns gained 20% there, but the branch
+            // cost its larger grids 2-3%.
+            constexpr bool FEW_COLS = T::NW == 1 && T::WTN <= 64;
+            if (FEW_COLS && nprog <= 8) {
+#pragma unroll
+              for (int t = h * NLDH; t < (h + 1) * NLDH; ++t) {
+                const int r = (t - h * NLDH) * T::F32_RPI + lane / T::F32_CPR;
+                const int cs = q ^ ((r / T::F32_RPP) % T::F32_XOR);
+                const f32x4 v = *(const TBK_LDS f32x4 *)(wl + r * T::F32_ROWB + cs * 16);
+                // computed here: off[t] (a whole block's offsets first) 0.5 us slower
+                const int row = row0 + h * BR + r;
+                // past the edges kOob, and out of range with 4 e added
+                const uint32_t aoff =
+                    (row < p.M && col < p.N)
+                        ? ((uint32_t)(row - m0) * (uint32_t)ld + (uint32_t)col) * 4u
+                        : kOob;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                  __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(v[e], rc, aoff + 4u * e, 0, 0);
+              }
+              continue;
+            }
             // one dword per lane, 64 consecutive columns (or 2 x 32) per
             // atomic: the atomics of a wave are served per cache line it
             // touches, and a lane's four columns as four atomics touched
@@ -1574,8 +1604,12 @@ __global__ __launch_bounds__(WGM *WGN * 64, 1) void gemm_kernel(GemmParams p) {
             // splits on one line at a time) measured 1 us slower, all splits
             // of a tile on one XCD 0.3-2 us slower.
             constexpr int NA = BR * T::WTN / 64; // dwords per lane per pass
-            // 8 at a time: unrolled whole, 8 waves of 64x128 ran out of registers
-#pragma unroll 8
+            // 8 at a time: unrolled whole, 8 waves of 64x128 ran out of registers.
+            // One wave of 64 columns has them for 32: 0-5% less per call from
+            // 16 workgroups to 2048^2 in 2 splits (64x64x64, 256^2 in 8: 7.88
+            // us to 7.54), none slower.
+            constexpr int UNROLL = FEW_COLS ? 32 : 8;
+#pragma unroll UNROLL
             for (int t = 0; t < NA; ++t) {
               const int r = (t * 64 + lane) / T::WTN; // row of the pass
               const int c = (t * 64 + lane) % T::WTN; // column of the wave tile

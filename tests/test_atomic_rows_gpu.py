@@ -1,6 +1,7 @@
 """Atomic split-K on wave tiles of 32, 64 and 128 columns, whose adds leave as
-64 consecutive dwords (two rows of 32, one of 64, half a row of 128), at the
-row and column edges: the result against f64, the padding columns unwritten.
+64 consecutive dwords (two rows of 32, one of 64, half a row of 128), or from
+a few workgroups of one 64-column wave as four dwords a lane, at the row and
+column edges: the result against f64, the padding columns unwritten.
 
 Bound per element: f32 products and sums in any order are off by at most
 (K + splits + 1) eps times the sum of the magnitudes added."""
@@ -15,11 +16,14 @@ pytestmark = pytest.mark.gpu
 
 # (block, wave grid): wave tiles of 32, 64 (16-row passes, then 32) and 128 columns
 TILES = [((64, 64, 64), (2, 2)), ((128, 64, 32), (4, 1)), ((128, 128, 64), (2, 2)),
-         ((256, 128, 64), (4, 1))]
+         ((256, 128, 64), (4, 1)),
+         # one wave: of 64 columns, 8 workgroups or fewer (with 3 splits one or two
+         # tiles) add four columns a lane and more whole lines; of 128 whole lines
+         ((64, 64, 32), (1, 1)), ((64, 128, 64), (1, 1))]
 
 
 @pytest.mark.parametrize("block,grid", TILES)
-@pytest.mark.parametrize("M,N", [(1, 8), (33, 136), (128, 128), (257, 72)])
+@pytest.mark.parametrize("M,N", [(1, 8), (33, 136), (40, 72), (128, 128), (257, 72)])
 def test_atomic_edges(block, grid, M, N, device):
     K, split, pad = 5 * block[2] + 8, 3, 8
     print(f"atomic {M}x{N}x{K} block {block} grid {grid}", flush=True)
